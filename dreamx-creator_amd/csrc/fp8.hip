@@ -269,7 +269,7 @@ __global__ __launch_bounds__(256) void quant_tensor_kernel(const T* __restrict__
 constexpr int GT = 256;                       // tile rows (M) and columns (N)
 constexpr int G_GROUP_M = 4;                  // M tiles per raster group
 
-struct GemmArgs {
+struct MatmulArgs {
   const uint8_t* a;      // [M, K]
   const uint8_t* b;      // [N, K]
   const float* sa;       // [1] or [M]
@@ -560,6 +560,36 @@ __device__ __forceinline__ uint32_t pos_key(uint32_t bits) {
   return (bits & 0x80000000u) ? 0u : bits;
 }
 
+// Four outputs of the epilogue rounded to bf16 (EPI 1: then their GELU, rounded
+// again), as two packed words.
+template <int EPI>
+__device__ __forceinline__ uint2 round_epilogue(const float v[4]) {
+  typedef float f32x2v __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2v __attribute__((ext_vector_type(2)));
+  bf16x2v p0 = __builtin_convertvector(f32x2v{v[0], v[1]}, bf16x2v);
+  bf16x2v p1 = __builtin_convertvector(f32x2v{v[2], v[3]}, bf16x2v);
+  if (EPI == 1) {
+    const uint32_t b0 = __builtin_bit_cast(uint32_t, p0), b1 = __builtin_bit_cast(uint32_t, p1);
+    const float r0 = __uint_as_float(b0 << 16), r1 = __uint_as_float(b0 & 0xffff0000u);
+    const float r2 = __uint_as_float(b1 << 16), r3 = __uint_as_float(b1 & 0xffff0000u);
+    p0 = __builtin_convertvector(f32x2v{gelu_tanh(r0), gelu_tanh(r1)}, bf16x2v);
+    p1 = __builtin_convertvector(f32x2v{gelu_tanh(r2), gelu_tanh(r3)}, bf16x2v);
+  }
+  return make_uint2(__builtin_bit_cast(uint32_t, p0), __builtin_bit_cast(uint32_t, p1));
+}
+
+// The amax word (AMAX 1: max |x|, 2: the largest positive value) raised by four
+// packed outputs.
+template <int AMAX>
+__device__ __forceinline__ uint32_t amax_of(uint2 p, uint32_t m) {
+  if (AMAX == 1) {
+    m = max(m, max((p.x & 0x7fffu) << 16, p.x & 0x7fff0000u));
+    return max(m, max((p.y & 0x7fffu) << 16, p.y & 0x7fff0000u));
+  }
+  m = max(m, max(pos_key(p.x << 16), pos_key(p.x & 0xffff0000u)));
+  return max(m, max(pos_key(p.y << 16), pos_key(p.y & 0xffff0000u)));
+}
+
 constexpr int G_FK = 128;                      // K bytes per fill stage
 constexpr int G_OPB = GT * G_FK;               // one operand tile of a stage: 32 KB
 constexpr int G_SLOT = 2 * G_OPB;              // 64 KB
@@ -584,7 +614,7 @@ struct GemmFrags {
 // cycles of the one fp8 MFMA they replace, so the data movement is unchanged.
 template <int EPI, int AMAX, int BF = 0, bool SPLIT = false>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
-void fp8_gemm_kernel(const GemmArgs g) {
+void fp8_gemm_kernel(const MatmulArgs g) {
   __shared__ __attribute__((aligned(1024))) uint8_t smem[G_LDS];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -884,26 +914,9 @@ void fp8_gemm_kernel(const GemmArgs g) {
           float v[4];
 #pragma unroll
           for (int r = 0; r < 4; ++r) v[r] = acc[i][j][4 * q + r] * sa * sb[r] + bias[r];
-          typedef float f32x2v __attribute__((ext_vector_type(2)));
-          typedef __bf16 bf16x2v __attribute__((ext_vector_type(2)));
-          bf16x2v p0 = __builtin_convertvector(f32x2v{v[0], v[1]}, bf16x2v);
-          bf16x2v p1 = __builtin_convertvector(f32x2v{v[2], v[3]}, bf16x2v);
-          if (EPI == 1) {
-            const uint32_t b0 = __builtin_bit_cast(uint32_t, p0), b1 = __builtin_bit_cast(uint32_t, p1);
-            const float r0_ = __uint_as_float(b0 << 16), r1_ = __uint_as_float(b0 & 0xffff0000u);
-            const float r2_ = __uint_as_float(b1 << 16), r3_ = __uint_as_float(b1 & 0xffff0000u);
-            p0 = __builtin_convertvector(f32x2v{gelu_tanh(r0_), gelu_tanh(r1_)}, bf16x2v);
-            p1 = __builtin_convertvector(f32x2v{gelu_tanh(r2_), gelu_tanh(r3_)}, bf16x2v);
-          }
-          const uint32_t px = __builtin_bit_cast(uint32_t, p0), py = __builtin_bit_cast(uint32_t, p1);
-          if (AMAX == 1 && mok && nok) {
-            amax = max(amax, max((px & 0x7fffu) << 16, px & 0x7fff0000u));
-            amax = max(amax, max((py & 0x7fffu) << 16, py & 0x7fff0000u));
-          } else if (AMAX == 2 && mok && nok) {
-            amax = max(amax, max(pos_key(px << 16), pos_key(px & 0xffff0000u)));
-            amax = max(amax, max(pos_key(py << 16), pos_key(py & 0xffff0000u)));
-          }
-          *reinterpret_cast<uint2*>(stg + mrow * 64 + 16 * (q ^ wswz) + 8 * hh) = make_uint2(px, py);
+          const uint2 px = round_epilogue<EPI>(v);
+          if (AMAX != 0 && mok && nok) amax = amax_of<AMAX>(px, amax);
+          *reinterpret_cast<uint2*>(stg + mrow * 64 + 16 * (q ^ wswz) + 8 * hh) = px;
         }
         // the 32 x 32 block back as 16 rows x 64 bytes per store
 #pragma unroll
@@ -927,6 +940,225 @@ void fp8_gemm_kernel(const GemmArgs g) {
     for (int i = 0; i < G_NI; ++i)
 #pragma unroll
       for (int j = 0; j < G_NJ; ++j) acc[i][j] = f32x16_t{};
+  }
+}
+
+// ------------------------------------------------ GEMM on small output tiles
+//
+// The same product for outputs that 256 x 256 tiles cannot spread over the
+// chip (the text projections' 512 rows: 24 such tiles on 256 CUs) and for the
+// last rows of a tall one (the 48 rows past 42 x 256 of a streamed chunk).
+// A workgroup of four wavefronts computes 64 MI rows x 64 columns; wavefront
+// (wm, wn) owns 32 MI rows x 32 columns.  A small grid is bound by the latency
+// and rate of its operand fetches (64 bytes per clock and CU), not by the
+// MFMAs, so operands stream through a ring of NST 128-byte K stages, all of them
+// in flight or being read, with one barrier a stage; a half-stage's fragments are
+// read while the half before it is multiplied.  LDS layout, fragment reads, MFMA
+// and K order are the large kernel's, so the results are the same bit for bit.
+// Tasks run column tile by column tile, contiguous per XCD, so the workgroups
+// of an XCD share weight rows in its L2 (and the few activation rows are in
+// each).  Rows past M and N read as zero through the buffer descriptor.
+//
+// A workgroup's fetches run at 60-65 GB/s (16 KB stages in 0.25 us), whatever
+// the ring's depth (3, 4, 5 or 8 stages within 5%), so three stages leave the
+// LDS for two (MI = 2) or three (MI = 1) workgroups per CU.  Measured against
+// 256 x 256 tiles, e4m3 operands, K = 3072, N = 3072: 48 rows 31.2 -> 7.8 us,
+// 512 rows 31.7 -> 10.0, 1024 rows 32.8 -> 17.3, 2048 rows 33.6 -> 29.3; bf16
+// operands against the register-fed kernel of dense.hip, 512 x 3072: K = 4096
+// 80.5 -> 24.7 us, K = 3072 63.6 -> 20.4 us.
+constexpr int GS_NST = 3;
+
+template <int EPI, int AMAX, int BF, int MI>
+__global__ __launch_bounds__(256) void small_tile_matmul_kernel(const MatmulArgs g) {
+  constexpr int TM = 64 * MI, TN = 64, NST = GS_NST;
+  constexpr int STAGE = (TM + TN) * G_FK;
+  constexpr int FILLS = 2 * MI + 2;  // fill DMAs per wavefront per stage
+  __shared__ __attribute__((aligned(1024))) uint8_t smem[NST * STAGE];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave & 1, wn = wave >> 1;
+  const uint32_t tiles_m = (uint32_t)(g.M + TM - 1) / TM;
+  const uint32_t task = xcd_task(blockIdx.x, gridDim.x);
+  const int m0 = (int)(task % tiles_m) * TM, n0 = (int)(task / tiles_m) * TN;
+  auto rsrc_of = [](const void* p, int64_t bytes) __attribute__((always_inline)) -> i32x4_t {
+    const uint64_t a = reinterpret_cast<uint64_t>(p);
+    return i32x4_t{static_cast<int>(static_cast<uint32_t>(a)),
+                   static_cast<int>(static_cast<uint32_t>(a >> 32)), static_cast<int>(bytes),
+                   0x00020000};
+  };
+  const i32x4_t ra = rsrc_of(g.a + (int64_t)m0 * g.K, (int64_t)(g.M - m0) * g.K);
+  const i32x4_t rb = rsrc_of(g.b + (int64_t)n0 * g.K, (int64_t)(g.N - n0) * g.K);
+  const uint32_t lds_base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(smem));
+  auto dma = [](i32x4_t rsrc, int voff, int soff, uint32_t lds) __attribute__((always_inline)) {
+    asm volatile("buffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(voff), "s"(rsrc), "s"(soff),
+                 "{m0}"(lds)
+                 : "memory");
+  };
+  // Fill: wavefront w writes activation rows [16 MI w, +16 MI) and weight rows
+  // [16 w, +16) of a stage, 8 rows of 128 bytes per DMA; lane l -> row 8 q + l/8,
+  // position l%8 holding source chunk (l%8) ^ ((row >> 1) & 7).
+  const int fpos = lane & 7;
+  const int sw_even = (fpos ^ ((lane >> 4) & 7)) * 16, sw_odd = (fpos ^ ((4 + (lane >> 4)) & 7)) * 16;
+  const int arow = (wave * 16 * MI + (lane >> 3)) * g.K;
+  const int brow = (wave * 16 + (lane >> 3)) * g.K;
+  auto fill = [&](int s, int slot) __attribute__((always_inline)) {
+    const uint32_t base = lds_base + slot * STAGE;
+    const int koff = s * G_FK;
+#pragma unroll
+    for (int q = 0; q < 2 * MI; ++q)
+      dma(ra, arow + q * 8 * g.K + ((q & 1) ? sw_odd : sw_even), koff,
+          base + (wave * 16 * MI + 8 * q) * G_FK);
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+      dma(rb, brow + q * 8 * g.K + ((q & 1) ? sw_odd : sw_even), koff,
+          base + (TM + wave * 16 + 8 * q) * G_FK);
+  };
+  const int rrow = lane & 31;
+  const int rswz = (rrow >> 1) & 7;
+  const int h2 = 2 * (lane >> 5);
+  int roff[2][2];
+#pragma unroll
+  for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) roff[kk][h] = rrow * G_FK + (((kk * 4 + h2 + h) ^ rswz) * 16);
+
+  f32x16_t acc[MI];
+#pragma unroll
+  for (int j = 0; j < MI; ++j) acc[j] = f32x16_t{};
+  struct Frags {
+    i32x8_t w, x[MI];
+  };
+  auto read = [&](int slot, auto kk_c) __attribute__((always_inline)) -> Frags {
+    constexpr int kk = decltype(kk_c)::value;
+    const uint8_t* ta = smem + slot * STAGE + wm * (32 * MI) * G_FK;
+    const uint8_t* tb = smem + slot * STAGE + (TM + wn * 32) * G_FK;
+    Frags f;
+    f.w = read_frag(tb, roff[kk][0], roff[kk][1]);
+#pragma unroll
+    for (int j = 0; j < MI; ++j) f.x[j] = read_frag(ta + j * 32 * G_FK, roff[kk][0], roff[kk][1]);
+    return f;
+  };
+  auto mma = [&](const Frags& f) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < MI; ++j) {
+      if constexpr (BF) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const i32x4_t wv = h ? __builtin_shufflevector(f.w, f.w, 4, 5, 6, 7)
+                               : __builtin_shufflevector(f.w, f.w, 0, 1, 2, 3);
+          const i32x4_t xv = h ? __builtin_shufflevector(f.x[j], f.x[j], 4, 5, 6, 7)
+                               : __builtin_shufflevector(f.x[j], f.x[j], 0, 1, 2, 3);
+          acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+              __builtin_bit_cast(bf16x8_t, wv), __builtin_bit_cast(bf16x8_t, xv), acc[j], 0, 0, 0);
+        }
+      } else {
+        acc[j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(f.w, f.x[j], acc[j], 0, 0, 0, 0,
+                                                                 0, 0);
+      }
+    }
+  };
+  using K0 = std::integral_constant<int, 0>;
+  using K1 = std::integral_constant<int, 1>;
+  const int nks = g.K / G_FK;
+#pragma unroll
+  for (int s = 0; s < NST; ++s)
+    if (s < nks) fill(s, s);
+  compiler_fence_gemm();
+  if (NST <= nks) waitcnt_vm<(NST - 1) * FILLS>();  // stage 0 landed
+  else waitcnt_vm<0>();
+  __builtin_amdgcn_s_barrier();
+  compiler_fence_gemm();
+  Frags f0 = read(0, K0{});
+  int slot = 0;
+  for (int s = 0; s < nks; ++s) {
+    // the stage's second half is read while its first is multiplied
+    const Frags f1 = read(slot, K1{});
+    __builtin_amdgcn_sched_barrier(0);
+    mma(f0);
+    __builtin_amdgcn_sched_barrier(0);
+    // stage s + 1 landed (this wavefront's fills; after the barrier everyone's);
+    // stage s is in registers everywhere, so its slot takes stage s + NST
+    compiler_fence_gemm();
+    if (s + NST - 1 < nks) waitcnt_vm<(NST - 2) * FILLS>();
+    else waitcnt_vm<0>();
+    __builtin_amdgcn_s_barrier();
+    compiler_fence_gemm();
+    if (s + NST < nks) fill(s + NST, slot);
+    slot = slot == NST - 1 ? 0 : slot + 1;
+    f0 = read(slot, K0{});  // after the last stage: stale data, not used
+    __builtin_amdgcn_sched_barrier(0);
+    mma(f1);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  // every wavefront is done with the ring: its first 8 KB hold the transposes
+  compiler_fence_gemm();
+  waitcnt_vm<0>();
+  __builtin_amdgcn_s_barrier();
+  compiler_fence_gemm();
+
+  const int rows = min(TM, g.M - m0);
+  int64_t obase = (int64_t)m0 * g.ldo;
+  if (g.split_n) obase += (int64_t)(n0 / g.split_n) * (g.split_stride - g.split_n);
+  const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)(g.out + obase), (short)0, (int)(((int64_t)(rows - 1) * g.ldo + g.N) * 2), 0x00020000);
+  const int hh = lane >> 5;
+  const int nw = n0 + wn * 32;  // the wavefront's first column
+  float sb[4][4], bias[4][4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int n = nw + 8 * q + 4 * hh;
+    const bool nok = n < g.N;
+    float4 v = make_float4(1.f, 1.f, 1.f, 1.f);
+    if (!BF) {
+      if (g.sb_per_col) {
+        if (nok) v = *reinterpret_cast<const float4*>(g.sb + n);
+      } else {
+        const float t = g.sb[0];
+        v = make_float4(t, t, t, t);
+      }
+    }
+    sb[q][0] = v.x; sb[q][1] = v.y; sb[q][2] = v.z; sb[q][3] = v.w;
+    uint2 bv = make_uint2(0u, 0u);
+    if (g.bias && nok) bv = *reinterpret_cast<const uint2*>(g.bias + n);
+    bias[q][0] = __uint_as_float(bv.x << 16);
+    bias[q][1] = __uint_as_float(bv.x & 0xffff0000u);
+    bias[q][2] = __uint_as_float(bv.y << 16);
+    bias[q][3] = __uint_as_float(bv.y & 0xffff0000u);
+  }
+  uint8_t* stg = smem + wave * 2048;
+  const int wswz = (rrow >> 1) & 3;
+  const int rb_row = lane >> 2, rb_c = lane & 3;
+  uint32_t amax = 0;
+#pragma unroll
+  for (int j = 0; j < MI; ++j) {
+    const int ml_w = wm * (32 * MI) + j * 32 + rrow;
+    const bool mok = ml_w < rows;
+    const float sa = BF ? 1.f : (g.sa_per_row ? (mok ? g.sa[m0 + ml_w] : 0.f) : g.sa[0]);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const bool nok = nw + 8 * q + 4 * hh < g.N;
+      float v[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] = acc[j][4 * q + r] * sa * sb[q][r] + bias[q][r];
+      const uint2 p = round_epilogue<EPI>(v);
+      if (AMAX != 0 && mok && nok) amax = amax_of<AMAX>(p, amax);
+      *reinterpret_cast<uint2*>(stg + rrow * 64 + 16 * (q ^ wswz) + 8 * hh) = p;
+    }
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+      const int rr = 16 * p + rb_row;
+      const i32x4_t d =
+          *reinterpret_cast<const i32x4_t*>(stg + rr * 64 + 16 * (rb_c ^ ((rr >> 1) & 3)));
+      const int ml = wm * (32 * MI) + j * 32 + rr;
+      const int n = nw + 8 * rb_c;
+      const int off = (n < g.N && ml < rows) ? (int)((ml * g.ldo + n) * 2) : (int)0x80000000;
+      __builtin_amdgcn_raw_buffer_store_b128(d, ro, off, 0, 0);
+    }
+  }
+  if (AMAX != 0) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) amax = max(amax, (uint32_t)__shfl_xor((int)amax, o));
+    if (lane == 0) raise_max_word(g.amax_out, amax);
   }
 }
 
@@ -1053,6 +1285,32 @@ TailSplit plan_tail_split(int64_t tiles, int64_t grid, int nks, int64_t max_unit
   return p;
 }
 
+// Which GEMMs run on 128 x 64 or 64 x 64 tiles (small_tile_matmul_kernel): those
+// with at most three 128 x 64 tiles per CU, that is, with under 0.4 of a round of
+// 256 x 256 tiles; 64 x 64 tiles up to two per CU.  Measured, K = 3072, us by
+// 64 x 64, 128 x 64 and 256 x 256 tiles: 512 x 3072 (1.5 tiles of 64 x 64 per CU)
+// 10.0, 12.4, 31.7; 1024 x 3072 (3) 17.4, 17.3, 32.8; 2048 x 3072 (6) 40.6,
+// 29.3, 33.6; 512 x 14336 (7) 35.2, 34.0, 34.0; 4096 x 3072 (12) 89, 86, 37.6.
+// Returns MI (tile rows / 64), 0 for 256 x 256 tiles.
+int small_tile_rows(int64_t M, int64_t N, int64_t cus) {
+  const int64_t tn = (N + 63) / 64;
+  if ((M + 63) / 64 * tn <= 2 * cus) return 1;
+  return (M + 127) / 128 * tn <= 3 * cus ? 2 : 0;
+}
+
+// The rows to leave to small tiles when the last, partial tile row of 256 x 256
+// tiles opens a round of its own (10800 x 3072: 516 tiles, the 12 of the last
+// 48 rows in a third round of 256 CUs): that round costs a whole tile's K loop
+// (27 us at K = 3072), the same rows on 64 x 64 tiles 8 us (240 rows: 8-9 us;
+// K = 14336: 27 us).  0 where the round stays, the rows would not be a small
+// grid, or the K loop is too short to pay for a second launch.
+int64_t remainder_rows(int64_t M, int64_t N, int64_t grid, int64_t cus, int nks) {
+  const int64_t rem = M % GT, tn = (N + GT - 1) / GT, full = M / GT * tn;
+  if (rem == 0 || full == 0 || nks < 8) return 0;
+  if ((full + grid - 1) / grid == (full + tn + grid - 1) / grid) return 0;
+  return small_tile_rows(rem, N, cus) == 1 ? rem : 0;
+}
+
 // Split-K workspace: one arrival counter per tail tile (left 0 by every
 // launch), then the partials, G_PART_BYTES per workgroup of the split launch.
 constexpr int64_t WS_COUNTERS = 4096;
@@ -1100,7 +1358,7 @@ int fp8_gemm_launch(const void* a, const void* b, const float* sa, int64_t sa_ro
                 epilogue);
   SRDIT_REQUIRE(!amax_pos || (amax_out && epilogue == 0),
                 "%s: SRDIT_GEMM_AMAX_POS needs amax_out and no GELU epilogue", who);
-  GemmArgs g;
+  MatmulArgs g;
   g.a = static_cast<const uint8_t*>(a);
   g.b = static_cast<const uint8_t*>(b);
   g.sa = sa;
@@ -1127,8 +1385,25 @@ int fp8_gemm_launch(const void* a, const void* b, const float* sa, int64_t sa_ro
     clear_u32_kernel<<<1, 1, 0, s>>>(amax_out);
     SRDIT_LAUNCH_CHECK("clear_u32_kernel");
   }
-  // one workgroup per CU, a multiple of 8 (one share per XCD), no more than the tiles need
   const int64_t cus = (cu_count_of_current_device() / 8) * 8;
+  auto launch_small = [&](const MatmulArgs& ga, auto mi_c) -> int {
+    constexpr int MI = decltype(mi_c)::value;
+    const int64_t n = (ga.M + 64 * MI - 1) / (64 * MI) * ((ga.N + 63) / 64);
+    const unsigned nwg = (unsigned)n;
+    if (bf16 && epilogue == 0) small_tile_matmul_kernel<0, 0, 1, MI><<<nwg, 256, 0, s>>>(ga);
+    else if (bf16) small_tile_matmul_kernel<1, 0, 1, MI><<<nwg, 256, 0, s>>>(ga);
+    else if (epilogue == 0 && !amax_out) small_tile_matmul_kernel<0, 0, 0, MI><<<nwg, 256, 0, s>>>(ga);
+    else if (epilogue == 0 && amax_pos) small_tile_matmul_kernel<0, 2, 0, MI><<<nwg, 256, 0, s>>>(ga);
+    else if (epilogue == 0) small_tile_matmul_kernel<0, 1, 0, MI><<<nwg, 256, 0, s>>>(ga);
+    else if (!amax_out) small_tile_matmul_kernel<1, 0, 0, MI><<<nwg, 256, 0, s>>>(ga);
+    else small_tile_matmul_kernel<1, 1, 0, MI><<<nwg, 256, 0, s>>>(ga);
+    SRDIT_LAUNCH_CHECK("small_tile_matmul_kernel");
+    return SRDIT_OK;
+  };
+  const int mi = small_tile_rows(M, N, cus);
+  if (mi == 1) return launch_small(g, std::integral_constant<int, 1>{});
+  if (mi == 2) return launch_small(g, std::integral_constant<int, 2>{});
+  // one workgroup per CU, a multiple of 8 (one share per XCD), no more than the tiles need
   const int64_t need = (tiles + 7) / 8 * 8;
   unsigned grid = (unsigned)(cus >= 8 ? (need < cus ? need : cus) : 8);
   const int64_t max_units =
@@ -1136,7 +1411,19 @@ int fp8_gemm_launch(const void* a, const void* b, const float* sa, int64_t sa_ro
   const TailSplit ts = max_units >= 2 && !bf16
                            ? plan_tail_split(tiles, grid, g.K / G_FK, max_units)
                            : TailSplit{};
-  auto launch = [&](const GemmArgs& ga, unsigned nwg, auto split_c) {
+  const int64_t rem = ts.split ? 0 : remainder_rows(M, N, grid, cus, g.K / G_FK);
+  if (rem) {  // the last rows on small tiles, the whole tile rows below
+    MatmulArgs r = g;
+    const int64_t m0 = M - rem;
+    r.a += m0 * g.K;
+    if (g.sa_per_row) r.sa += m0;
+    r.out += m0 * ldo;
+    r.M = (int)rem;
+    if (int rc = launch_small(r, std::integral_constant<int, 1>{})) return rc;
+    g.M = (int)m0;
+    g.tiles_m = (int)(m0 / GT);
+  }
+  auto launch = [&](const MatmulArgs& ga, unsigned nwg, auto split_c) {
     constexpr bool SP = decltype(split_c)::value;
     if (bf16 && epilogue == 0) fp8_gemm_kernel<0, 0, 1><<<nwg, 512, 0, s>>>(ga);
     else if (bf16) fp8_gemm_kernel<1, 0, 1><<<nwg, 512, 0, s>>>(ga);
@@ -1148,7 +1435,7 @@ int fp8_gemm_launch(const void* a, const void* b, const float* sa, int64_t sa_ro
   };
   // the whole rounds (every tile when nothing is split)
   g.task_base = 0;
-  g.n_tasks = (int)(tiles - ts.tail);
+  g.n_tasks = g.tiles_m * g.tiles_n - ts.tail;
   g.split_k = 0;
   g.ws_part = nullptr;
   g.ws_cnt = nullptr;
