@@ -344,6 +344,287 @@ __global__ __launch_bounds__(256) void linear_f32_modulated_kernel(
 }
 
 // ---------------------------------------------------------------------------
+// The same product for bf16 weights on bf16 MFMAs, without rounding anything the
+// fp32 MFMAs keep: xin is cut into three bf16 pieces of 8 significant bits each
+// (its leading bits, those of the remainder, and the rest, all exact), every
+// product of a piece with a bf16 weight is exact in fp32, and the sums stay fp32
+// (the leading pieces in one accumulator, the others in a second).  An infinite
+// xin keeps its infinity in the leading piece and zeros in the others; a NaN
+// stays one.  Three bf16 MFMAs do the work of sixteen times as many fp32 ones.
+//
+// A workgroup owns 64 rows and 32 NT columns.  Its eight wavefronts are two row
+// halves times four slices of 16 k in every 64-k stage, so each element of xin is
+// formed and cut once and two wavefronts share a SIMD; the slices' sums meet in
+// LDS at the end, in slice order.  Stages (128-byte rows, 16-byte chunk c of row r
+// at c ^ ((r >> 1) & 7), which keeps the fragment reads of 16 lanes on distinct
+// banks) stream through a ring of HM_NST; the next stage's fragments are read and
+// cut while this one is multiplied.  s1 and m0 sit in LDS for the whole walk.  The
+// weights are the MFMA's first operand: a lane holds runs of four columns of one row.
+// Bound by its own chain: about 0.97 us per stage, 0.55 of it MFMAs (one workgroup
+// per CU, 169 of them at 10800 rows); without the cut it is 0.82 us.
+// Measured against the fp32 MFMAs, N = 192, K = 3072: 10800 rows 124.5 -> 59.0 us,
+// 21600 rows 227.6 -> 115.6, 3000 rows 62.2 -> 54.8; relative error against 64
+// bits 4.0e-7 -> 2.4e-7 (the sums are four chains of 48 x 3 additions, not of 384).
+constexpr int HM_NST = 3;
+constexpr int HM_ROWS = 64;
+constexpr int HM_MAX_K = 4096;  // s1 and m0 take 8 K bytes of LDS
+
+// Where s1 and m0 come from: given, or (mod != null) the head's adaLN vectors
+// m0 = f32(mod[0]) + e and s1 = 1 + (f32(mod[1]) + e), rounded after each sum.
+struct ModSource {
+  const float* s1;
+  const float* m0;
+  const void* mod;  // [2, K], bf16 or fp32
+  const float* e;   // [K]
+  int mod_bf16;
+};
+
+__device__ __forceinline__ i32x4_t raw_rsrc(const void* p, int64_t bytes) {
+  const uint64_t a = reinterpret_cast<uint64_t>(p);
+  return i32x4_t{static_cast<int>(static_cast<uint32_t>(a)),
+                 static_cast<int>(static_cast<uint32_t>(a >> 32)), static_cast<int>(bytes),
+                 0x00020000};
+}
+
+// 16 bytes per lane to LDS at lds + 16 lane; the compiler does not see the LDS
+// write, so callers wait and synchronise before they read it.
+__device__ __forceinline__ void dma16(i32x4_t rsrc, int voff, int soff, uint32_t lds) {
+  asm volatile("buffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(voff), "s"(rsrc), "s"(soff),
+               "{m0}"(lds)
+               : "memory");
+}
+
+// At most N vector-memory operations in flight, LDS reads retired, then a barrier.
+template <int N>
+__device__ __forceinline__ void stage_barrier() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4));
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+struct Cut3 {
+  bf16x8_t hi, mid, lo;
+};
+
+__device__ __forceinline__ uint32_t top_halves(float a, float b) {
+  return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
+}
+
+// Eight bf16 of a row -> xin -> its three pieces.
+__device__ __forceinline__ Cut3 modulate_cut(const i32x4_t a, const float* s1, const float* m0) {
+#pragma clang fp contract(off)
+  i32x4_t hi, mid, lo;
+#pragma unroll
+  for (int p = 0; p < 4; ++p) {
+    const uint32_t w = static_cast<uint32_t>(a[p]);
+    float x[2] = {__uint_as_float(w << 16), __uint_as_float(w & 0xffff0000u)};
+    float r[2], t[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      x[i] = x[i] * s1[2 * p + i] + m0[2 * p + i];
+      const float h = __uint_as_float(__float_as_uint(x[i]) & 0xffff0000u);
+      r[i] = __builtin_fabsf(x[i]) == INFINITY ? 0.f : x[i] - h;
+      t[i] = r[i] - __uint_as_float(__float_as_uint(r[i]) & 0xffff0000u);
+    }
+    hi[p] = static_cast<int>(top_halves(x[0], x[1]));
+    mid[p] = static_cast<int>(top_halves(r[0], r[1]));
+    lo[p] = static_cast<int>(top_halves(t[0], t[1]));
+  }
+  return Cut3{__builtin_bit_cast(bf16x8_t, hi), __builtin_bit_cast(bf16x8_t, mid),
+              __builtin_bit_cast(bf16x8_t, lo)};
+}
+
+template <int NT>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void linear_f32_cut_kernel(const uint16_t* __restrict__ a, int64_t lda, ModSource ms,
+                           const uint16_t* __restrict__ w, int64_t ldw,
+                           const uint16_t* __restrict__ bias, float* __restrict__ out, int64_t ldo,
+                           int M, int N, int K, bool vec_out) {
+  constexpr int KB = 128;                          // bytes of k per stage
+  constexpr int STAGE = (32 * NT + HM_ROWS) * KB;
+  constexpr int WD = NT / 2;                       // weight DMAs per wavefront per stage
+  constexpr int FILLS = WD + 1;
+  constexpr int PART = 32 * 32 * NT;               // floats of one wavefront's sums
+  constexpr int RING = HM_NST * STAGE > 4 * PART * 4 ? HM_NST * STAGE : 4 * PART * 4;
+  __shared__ __attribute__((aligned(1024))) uint8_t smem[RING + 8 * HM_MAX_K];
+  float* ls1 = reinterpret_cast<float*>(smem + RING);
+  float* lm0 = ls1 + K;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int half = wave & 1, slice = wave >> 1;
+  const int m_base = blockIdx.y * HM_ROWS, n_base = blockIdx.x * 32 * NT;
+
+  // Rows past the end read as zero through the descriptors' range check.
+  const int rows = min(HM_ROWS, M - m_base), cols = min(32 * NT, N - n_base);
+  const i32x4_t ra = raw_rsrc(a + (int64_t)m_base * lda, ((int64_t)(rows - 1) * lda + K) * 2);
+  const i32x4_t rw = raw_rsrc(w + (int64_t)n_base * ldw, ((int64_t)(cols - 1) * ldw + K) * 2);
+  const uint32_t lds_base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(smem));
+  // A DMA writes 8 rows of 128 bytes: lane l -> row l/8, position l%8 holding source
+  // chunk (l%8) ^ ((row >> 1) & 7).  Wavefront w: activation rows [8 w, +8) and
+  // weight rows [8 WD w, +8 WD).
+  const int fr = lane >> 3, fp = lane & 7;
+  auto fill = [&](int s, int slot) __attribute__((always_inline)) {
+    const uint32_t base = lds_base + slot * STAGE;
+#pragma unroll
+    for (int q = 0; q < WD; ++q) {
+      const int r = wave * 8 * WD + 8 * q + fr;
+      const int off = r < cols ? (int)(r * ldw * 2) + ((fp ^ ((r >> 1) & 7)) * 16) : (int)0x80000000;
+      dma16(rw, off, s * KB, base + (wave * 8 * WD + 8 * q) * KB);
+    }
+    const int r = wave * 8 + fr;
+    const int off = r < rows ? (int)(r * lda * 2) + ((fp ^ ((r >> 1) & 7)) * 16) : (int)0x80000000;
+    dma16(ra, off, s * KB, base + (32 * NT + wave * 8) * KB);
+  };
+  const int nst = K / 64;
+#pragma unroll
+  for (int s = 0; s < HM_NST; ++s)
+    if (s < nst) fill(s, s);
+  for (int k = threadIdx.x; k < K; k += 512) {
+    if (ms.mod) {
+      const float b0 = ms.mod_bf16 ? bf16_bits_to_f32(static_cast<const uint16_t*>(ms.mod)[k])
+                                   : static_cast<const float*>(ms.mod)[k];
+      const float b1 = ms.mod_bf16 ? bf16_bits_to_f32(static_cast<const uint16_t*>(ms.mod)[K + k])
+                                   : static_cast<const float*>(ms.mod)[K + k];
+      ls1[k] = 1.f + (b1 + ms.e[k]);
+      lm0[k] = b0 + ms.e[k];
+    } else {
+      ls1[k] = ms.s1[k];
+      lm0[k] = ms.m0[k];
+    }
+  }
+
+  // Fragments of this wavefront's 16 k: lane l holds row l%32, k 8 (l/32) .. +8:
+  // chunk 2 slice + l/32 of the row.
+  const int frow = lane & 31, fg = lane >> 5;
+  const int foff = frow * KB + (((2 * slice + fg) ^ ((frow >> 1) & 7)) * 16);
+  const int kl = 16 * slice + 8 * fg;
+  struct Frag {
+    bf16x8_t w[NT];
+    Cut3 x;
+  };
+  struct Raw {
+    i32x4_t a;
+    float s1[8], m0[8];
+  };
+  auto read = [&](int s, int slot, bf16x8_t (&wf)[NT]) __attribute__((always_inline)) -> Raw {
+    const uint8_t* base = smem + slot * STAGE + foff;
+    Raw r;
+    r.a = *reinterpret_cast<const i32x4_t*>(base + (32 * NT + 32 * half) * KB);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const f32x4_t s4 = *reinterpret_cast<const f32x4_t*>(ls1 + 64 * s + kl + 4 * h);
+      const f32x4_t m4 = *reinterpret_cast<const f32x4_t*>(lm0 + 64 * s + kl + 4 * h);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) { r.s1[4 * h + i] = s4[i]; r.m0[4 * h + i] = m4[i]; }
+    }
+#pragma unroll
+    for (int t = 0; t < NT; ++t) wf[t] = *reinterpret_cast<const bf16x8_t*>(base + 32 * t * KB);
+    return r;
+  };
+  f32x16_t acc[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) acc[t] = f32x16_t{};
+  auto mma = [&](const Frag& f) __attribute__((always_inline)) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+      acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.w[t], f.x.lo, acc[t], 0, 0, 0);
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+      acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.w[t], f.x.mid, acc[t], 0, 0, 0);
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+      acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.w[t], f.x.hi, acc[t], 0, 0, 0);
+  };
+  __syncthreads();   // s1 and m0 are written
+  stage_barrier<0>();  // the first stages landed
+  Frag f0;
+  {
+    const Raw r = read(0, 0, f0.w);
+    f0.x = modulate_cut(r.a, r.s1, r.m0);
+  }
+  int slot = 0;
+  auto step = [&](int s, const Frag& fc, Frag& fn) __attribute__((always_inline)) {
+    // stage s + 1 landed everywhere; stage s is in registers, its slot takes s + NST
+    if (s + HM_NST - 1 < nst) stage_barrier<(HM_NST - 2) * FILLS>();
+    else stage_barrier<0>();
+    if (s + HM_NST < nst) fill(s + HM_NST, slot);
+    slot = slot == HM_NST - 1 ? 0 : slot + 1;
+    const Raw r = read(s + 1 < nst ? s + 1 : s, slot, fn.w);  // after the last stage: not used
+    __builtin_amdgcn_sched_barrier(0);
+    mma(fc);
+    fn.x = modulate_cut(r.a, r.s1, r.m0);
+    // the first MFMAs cover the reads' latency; the cut's vector operations then
+    // fill the matrix pipe's 32 cycles per MFMA
+    __builtin_amdgcn_sched_group_barrier(0x008, NT, 0);     // MFMAs
+#pragma unroll
+    for (int i = 0; i < 2 * NT; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
+      __builtin_amdgcn_sched_group_barrier(0x002, 9, 0);  // nine VALU
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  Frag f1;
+  int s = 0;
+  for (; s + 1 < nst; s += 2) {
+    step(s, f0, f1);
+    step(s + 1, f1, f0);
+  }
+  if (s < nst) step(s, f0, f1);
+
+  // The slices' sums: 2 and 3 to LDS, 0 and 1 add them; then 1 to LDS and 0 adds it.
+  stage_barrier<0>();
+  f32x4_t* part = reinterpret_cast<f32x4_t*>(smem);
+  auto at = [&](int p, int t, int g) __attribute__((always_inline)) -> f32x4_t& {
+    return part[((p * NT + t) * 4 + g) * 64 + lane];
+  };
+#pragma unroll
+  for (int round = 0; round < 2; ++round) {
+    const int lo = round == 0 ? 2 : 1;  // slices [lo, 2 lo) are written, [0, lo) add them
+    if (slice >= lo && slice < 2 * lo) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+          at(2 * (slice - lo) + half, t, g) =
+              f32x4_t{acc[t][4 * g], acc[t][4 * g + 1], acc[t][4 * g + 2], acc[t][4 * g + 3]};
+    }
+    __syncthreads();
+    if (slice < lo) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const f32x4_t v = at(2 * slice + half, t, g);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) acc[t][4 * g + i] += v[i];
+        }
+    }
+    __syncthreads();
+  }
+  // lane l: row l%32 of the half, columns 32 t + 8 g + 4 (l/32) .. +4
+  const int m = m_base + 32 * half + frow;
+  if (slice != 0 || m >= M) return;
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const int n = n_base + 32 * t + 8 * g + 4 * fg;
+      float* dst = out + (int64_t)m * ldo + n;
+      f32x4_t v = {acc[t][4 * g], acc[t][4 * g + 1], acc[t][4 * g + 2], acc[t][4 * g + 3]};
+      if (n + 4 <= N && vec_out) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] += bias ? bf16_bits_to_f32(bias[n + i]) : 0.f;
+        *reinterpret_cast<f32x4_t*>(dst) = v;
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (n + i < N) dst[i] = v[i] + (bias ? bf16_bits_to_f32(bias[n + i]) : 0.f);
+      }
+    }
+}
+
+// ---------------------------------------------------------------------------
 // fp32 GEMV rows: out[m, n] = sum_k x[m, k] w[n, k] + b[n].  One wave per
 // output (4 per workgroup); the lanes stride the row 8 elements at a time and
 // the 64 partial sums reduce across the wave.
@@ -389,6 +670,34 @@ int pick_ks(int64_t M, int64_t N, int64_t K) {
   const int64_t tiles = ((M + 4 * WT_M - 1) / (4 * WT_M)) * ((N + WT_N - 1) / WT_N);
   const int64_t steps = K / 16;
   return (steps % 4 == 0 && steps >= 16 && tiles < 512) ? 4 : 1;
+}
+
+// bf16 weights over whole 64-k stages with s1 and m0 in LDS: the cut-operand kernel
+// can take them.
+bool cut_fits(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldw, int w_dtype) {
+  return w_dtype == SRDIT_DTYPE_BF16 && K % 64 == 0 && K <= HM_MAX_K &&
+         M <= 65535LL * HM_ROWS && HM_ROWS * lda * 2 < (1LL << 31) && 192 * ldw * 2 < (1LL << 31);
+}
+
+// It takes about 52 us for up to 256 workgroups (K = 3072, N = 192), the fp32
+// kernel 34 us below 1000 rows and 62 us at 3000; with 64 columns 31 us against
+// 34 at any row count.
+bool cut_pays(int64_t M, int64_t N) { return N <= 64 || M * ((N + 191) / 192) >= 2560; }
+
+void launch_cut(const void* a, int64_t lda, const ModSource& ms, const void* w, int64_t ldw,
+                const void* bias, float* out, int64_t ldo, int64_t M, int64_t N, int64_t K,
+                hipStream_t s) {
+  const bool vec_out = aligned_rows16(out, ldo, 4);
+  const uint16_t* ap = static_cast<const uint16_t*>(a);
+  const uint16_t* wp = static_cast<const uint16_t*>(w);
+  const uint16_t* bp = static_cast<const uint16_t*>(bias);
+  const unsigned gy = (unsigned)((M + HM_ROWS - 1) / HM_ROWS);
+  if (N <= 64)
+    linear_f32_cut_kernel<2><<<dim3(1, gy), 512, 0, s>>>(ap, lda, ms, wp, ldw, bp, out, ldo,
+                                                         (int)M, (int)N, (int)K, vec_out);
+  else
+    linear_f32_cut_kernel<6><<<dim3((unsigned)((N + 191) / 192), gy), 512, 0, s>>>(
+        ap, lda, ms, wp, ldw, bp, out, ldo, (int)M, (int)N, (int)K, vec_out);
 }
 
 dim3 dense_grid(int64_t M, int64_t N, int ks) {
@@ -468,10 +777,15 @@ extern "C" int srdit_linear_f32_modulated(const void* a, int64_t lda, const floa
                     (!bias || (reinterpret_cast<uintptr_t>(bias) & (welem - 1)) == 0),
                 "%s: misaligned output or bias", fn);
   const bool vec_out = aligned_rows16(out, ldo, 4);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  if (cut_fits(M, N, K, lda, ldw, w_dtype) && cut_pays(M, N)) {
+    launch_cut(a, lda, ModSource{s1, m0, nullptr, nullptr, 0}, w, ldw, bias, out, ldo, M, N, K, s);
+    SRDIT_LAUNCH_CHECK("linear_f32_cut_kernel");
+    return SRDIT_OK;
+  }
   const int ks = pick_ks(M, N, K);
   const dim3 grid = dense_grid(M, N, ks);
   SRDIT_REQUIRE(grid.y < 65536u * 16, "%s: M=%lld too large", fn, (long long)M);
-  hipStream_t s = static_cast<hipStream_t>(stream);
   const uint16_t* ap = static_cast<const uint16_t*>(a);
 #define SRDIT_LF(WT, KS)                                                                        \
   linear_f32_modulated_kernel<WT, KS><<<grid, 256, 0, s>>>(ap, lda, s1, m0,                     \
@@ -484,6 +798,35 @@ extern "C" int srdit_linear_f32_modulated(const void* a, int64_t lda, const floa
   else SRDIT_LF(uint16_t, 1);
 #undef SRDIT_LF
   SRDIT_LAUNCH_CHECK("linear_f32_modulated_kernel");
+  return SRDIT_OK;
+}
+
+extern "C" int srdit_head_linear(const void* a, int64_t lda, const void* mod, int mod_dtype,
+                                 const float* e, const void* w, int64_t ldw, const void* bias,
+                                 float* out, int64_t ldo, int64_t M, int64_t N, int64_t K,
+                                 void* stream) {
+  const char* fn = "srdit_head_linear";
+  SRDIT_REQUIRE(a && mod && e && w && out, "%s: null operand", fn);
+  SRDIT_REQUIRE(mod_dtype == SRDIT_DTYPE_BF16 || mod_dtype == SRDIT_DTYPE_FP32,
+                "%s: mod_dtype %d is not bf16 (0) or fp32 (2)", fn, mod_dtype);
+  SRDIT_REQUIRE(M > 0 && N > 0 && K > 0 && M < (1LL << 31) && N < (1LL << 31) && K < (1LL << 31),
+                "%s: bad sizes M=%lld N=%lld K=%lld", fn, (long long)M, (long long)N,
+                (long long)K);
+  SRDIT_REQUIRE(lda >= K && ldw >= K && ldo >= N, "%s: leading dimensions below the row length",
+                fn);
+  SRDIT_REQUIRE(cut_fits(M, N, K, lda, ldw, SRDIT_DTYPE_BF16),
+                "%s: K=%lld must be a multiple of 64, at most %d, and the rows below 2^31 bytes", fn,
+                (long long)K, HM_MAX_K);
+  SRDIT_REQUIRE(aligned_rows16(a, lda, 2) && aligned_rows16(w, ldw, 2),
+                "%s: A and W rows must be 16-byte aligned", fn);
+  SRDIT_REQUIRE((reinterpret_cast<uintptr_t>(out) & 3) == 0 &&
+                    (reinterpret_cast<uintptr_t>(e) & 3) == 0 &&
+                    (reinterpret_cast<uintptr_t>(mod) & 3) == 0 &&
+                    (!bias || (reinterpret_cast<uintptr_t>(bias) & 1) == 0),
+                "%s: misaligned vector or output", fn);
+  launch_cut(a, lda, ModSource{nullptr, nullptr, mod, e, mod_dtype == SRDIT_DTYPE_BF16}, w, ldw,
+             bias, out, ldo, M, N, K, static_cast<hipStream_t>(stream));
+  SRDIT_LAUNCH_CHECK("linear_f32_cut_kernel");
   return SRDIT_OK;
 }
 

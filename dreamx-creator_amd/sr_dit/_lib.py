@@ -73,6 +73,8 @@ SIGNATURES = {
                                    _c_i64, _c_i64, _c_int, _c_p]),
     "srdit_linear_f32_modulated": (_c_int, [_c_p, _c_i64, _c_p, _c_p, _c_p, _c_i64, _c_p, _c_int,
                                             _c_p, _c_i64, _c_i64, _c_i64, _c_i64, _c_p]),
+    "srdit_head_linear": (_c_int, [_c_p, _c_i64, _c_p, _c_int, _c_p, _c_p, _c_i64, _c_p, _c_p,
+                                   _c_i64, _c_i64, _c_i64, _c_i64, _c_p]),
     "srdit_gemv_f32": (_c_int, [_c_p, _c_i64, _c_p, _c_i64, _c_p, _c_int, _c_p, _c_i64, _c_i64,
                                 _c_i64, _c_i64, _c_p]),
     "srdit_last_error": (_c_int, [ctypes.c_char_p, _c_int]),
@@ -534,6 +536,37 @@ def linear_f32_modulated(a, s1, m0, w, bias, out):
                                            w.stride(0), _ptr(bias), _DENSE_W_CODES[w.dtype],
                                            _ptr(out), out.stride(0), M, N, K, _stream(a.device))
     _check(rc, "srdit_linear_f32_modulated")
+
+
+def head_linear_fits(rows, w, mod, e):
+    """Whether ``head_linear`` takes these weights [N, K], modulation [1, 2, K] and
+    timestep embedding [1, K], and is the faster call for ``rows`` rows (from 2560 on,
+    any number for up to 64 columns); ``linear_f32_modulated`` takes the rest."""
+    N, K = w.shape
+    return (w.dtype == torch.bfloat16 and K % 64 == 0 and K <= 4096
+            and (N <= 64 or rows * -(-N // 192) >= 2560)
+            and mod.dtype in _DENSE_W_CODES and mod.numel() == 2 * K and mod.is_contiguous()
+            and e.dtype == torch.float32 and e.numel() == K and e.is_contiguous())
+
+
+def head_linear(a, mod, e, w, bias, out):
+    """``linear_f32_modulated`` with bf16 weights, m0 = f32(mod[0]) + e and s1 = 1 +
+    (f32(mod[1]) + e) formed by the call: mod [1, 2, K] bf16 or fp32, e [1, K] fp32."""
+    _rows2d("head_linear a", a, torch.bfloat16)
+    _rows2d("head_linear w", w, torch.bfloat16)
+    _rows2d("head_linear out", out, torch.float32)
+    M, K = a.shape
+    N = w.shape[0]
+    if w.shape[1] != K or tuple(out.shape) != (M, N) or mod.dtype not in _DENSE_W_CODES:
+        raise ValueError(f"head_linear: a {tuple(a.shape)} w {tuple(w.shape)} out "
+                         f"{tuple(out.shape)} mod {tuple(mod.shape)} e {tuple(e.shape)} disagree")
+    _vec("head_linear mod", mod, 2 * K, mod.dtype)
+    _vec("head_linear e", e, K, torch.float32)
+    _vec("head_linear bias", bias, N, torch.bfloat16)
+    rc = load().srdit_head_linear(_ptr(a), a.stride(0), _ptr(mod), _DENSE_W_CODES[mod.dtype],
+                                  _ptr(e), _ptr(w), w.stride(0), _ptr(bias), _ptr(out),
+                                  out.stride(0), M, N, K, _stream(a.device))
+    _check(rc, "srdit_head_linear")
 
 
 def gemv_f32(x, w, bias, out):

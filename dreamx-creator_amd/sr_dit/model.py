@@ -589,11 +589,9 @@ class Head(nn.Module):
         """The same arithmetic in two kernels: the LayerNorm's bf16 output
         (srdit_ln_modulate without modulation), then the fp32 Linear that
         applies f32(ln) * (1 + scale) + shift to its input as it reads it
-        (srdit_linear_f32_modulated); the weights stay in their dtype (bf16 or
-        fp32), as .float() of them is exact."""
-        m = self.modulation.float() + e.float().unsqueeze(1)          # [1, 2, dim]
-        s1 = (1 + m[0, 1]).contiguous()
-        m0 = m[0, 0].contiguous()
+        (srdit_head_linear, which forms scale and shift too, for bf16 weights;
+        srdit_linear_f32_modulated otherwise); the weights stay in their dtype
+        (bf16 or fp32), as .float() of them is exact."""
         xb = x.contiguous()
         ln = torch.empty_like(xb)
         nw, nb = self.norm.weight, self.norm.bias
@@ -601,10 +599,15 @@ class Head(nn.Module):
             nw, nb = nw.to(torch.bfloat16).contiguous(), nb.to(torch.bfloat16).contiguous()
         _lib.ln_modulate(xb, nw, nb, None, None, self.norm.eps, ln)
         w = self.head.weight
-        w = w if w.dtype in (torch.bfloat16, torch.float32) else w.float()
+        w = (w if w.dtype in (torch.bfloat16, torch.float32) else w.float()).contiguous()
         b = None if self.head.bias is None else self.head.bias.to(w.dtype).contiguous()
         out = torch.empty(x.shape[0], w.shape[0], dtype=torch.float32, device=x.device)
-        _lib.linear_f32_modulated(ln, s1, m0, w.contiguous(), b, out)
+        if _lib.head_linear_fits(x.shape[0], w, self.modulation, e):
+            _lib.head_linear(ln, self.modulation, e, w, b, out)
+        else:
+            m = self.modulation.float() + e.float().unsqueeze(1)      # [1, 2, dim]
+            _lib.linear_f32_modulated(ln, (1 + m[0, 1]).contiguous(), m[0, 0].contiguous(), w, b,
+                                      out)
         return out
 
 

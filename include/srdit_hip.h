@@ -406,6 +406,16 @@ int srdit_linear_f32_modulated(const void* a, int64_t lda, const float* s1, cons
                                void* stream);
 
 /*
+ * srdit_linear_f32_modulated with bf16 w and bias (bias may be NULL) and the
+ * vectors formed by the call as Head.forward forms them: m0 = f32(mod[0]) + e and
+ * s1 = 1 + (f32(mod[1]) + e), mod [2, K] bf16 or fp32 (mod_dtype) and e fp32 [K],
+ * each sum rounded.  K % 64 == 0, K <= 4096.
+ */
+int srdit_head_linear(const void* a, int64_t lda, const void* mod, int mod_dtype, const float* e,
+                      const void* w, int64_t ldw, const void* bias, float* out, int64_t ldo,
+                      int64_t M, int64_t N, int64_t K, void* stream);
+
+/*
  * out [M, N] fp32 = x [M, K] fp32 @ w [N, K]^T + bias, w and bias both bf16 or
  * both fp32 (w_dtype), bias may be NULL; K % 8 == 0, M < 65536.  One wave per
  * output: for the time embedding's and time projection's Linears on the
