@@ -629,27 +629,67 @@ void linear_f32_cut_kernel(const uint16_t* __restrict__ a, int64_t lda, ModSourc
 // output (4 per workgroup); the lanes stride the row 8 elements at a time and
 // the 64 partial sums reduce across the wave.
 template <typename WT>
-__global__ __launch_bounds__(256) void gemv_f32_kernel(const float* __restrict__ x, int64_t ldx,
-                                                       const WT* __restrict__ w, int64_t ldw,
-                                                       const WT* __restrict__ bias,
-                                                       float* __restrict__ out, int64_t ldo,
-                                                       int N, int K) {
-  const int lane = threadIdx.x & 63;
-  const int n = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (n >= N) return;  // whole waves: no barrier follows
-  const int m = blockIdx.y;
-  const float* xr = x + (int64_t)m * ldx;
-  const WT* wr = w + (int64_t)n * ldw;
+__device__ __forceinline__ float wave_dot(const float* x, const WT* __restrict__ w, int K, int lane) {
   float acc = 0.f;
   for (int k = lane * 8; k < K; k += 512) {
-    const f32x8v xv = load8_f32<float>(xr + k);
-    const f32x8v wv = load8_f32<WT>(wr + k);
+    const f32x8v xv = load8_f32<float>(x + k);
+    const f32x8v wv = load8_f32<WT>(w + k);
 #pragma unroll
     for (int i = 0; i < 8; ++i) acc = __builtin_fmaf(xv[i], wv[i], acc);
   }
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) acc += __shfl_xor(acc, off);
-  if (lane == 0) out[(int64_t)m * ldo + n] = acc + (bias ? load1_f32<WT>(bias, n) : 0.f);
+  return acc;
+}
+
+// x / (1 + e^-x), as torch's fp32 silu.
+__device__ __forceinline__ float silu_f32(float x) { return x / (1.0f + expf(-x)); }
+
+// SILU: silu_out (beside out, which may be null) takes the result's silu.
+template <typename WT, bool SILU>
+__global__ __launch_bounds__(256) void gemv_f32_kernel(const float* __restrict__ x, int64_t ldx,
+                                                       const WT* __restrict__ w, int64_t ldw,
+                                                       const WT* __restrict__ bias,
+                                                       float* __restrict__ out, int64_t ldo,
+                                                       int N, int K, float* __restrict__ silu_out) {
+  const int lane = threadIdx.x & 63;
+  const int n = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (n >= N) return;  // whole waves: no barrier follows
+  const int m = blockIdx.y;
+  const float acc = wave_dot<WT>(x + (int64_t)m * ldx, w + (int64_t)n * ldw, K, lane);
+  if (lane == 0) {
+    const float v = acc + (bias ? load1_f32<WT>(bias, n) : 0.f);
+    if (out) out[(int64_t)m * ldo + n] = v;
+    if (SILU) silu_out[n] = silu_f32(v);
+  }
+}
+
+// silu of the time MLP's first Linear on the sinusoid of one timestep.  Every
+// workgroup forms the sinusoid in LDS, in 64 bits as the reference does (cos of
+// t 10000^(-i / half), then sin, rounded to fp32), and takes TE_OUT outputs per
+// wave, so that work is repeated 192 times at dim 3072, not 768.
+constexpr int TE_OUT = 4;
+constexpr int TE_MAX_FREQ = 2048;
+
+template <typename WT>
+__global__ __launch_bounds__(256) void time_sinusoid_gemv_kernel(
+    const float* __restrict__ t, int freq, const WT* __restrict__ w, const WT* __restrict__ bias,
+    float* __restrict__ silu_out, int N) {
+  __shared__ __attribute__((aligned(16))) float x[TE_MAX_FREQ];
+  const int half = freq / 2;
+  const double pos = static_cast<double>(t[0]);
+  for (int i = threadIdx.x; i < half; i += 256) {
+    const double ang = pos * pow(10000.0, -static_cast<double>(i) / static_cast<double>(half));
+    x[i] = static_cast<float>(cos(ang));
+    x[half + i] = static_cast<float>(sin(ang));
+  }
+  __syncthreads();
+  const int lane = threadIdx.x & 63;
+  const int n0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * TE_OUT;
+  for (int n = n0; n < min(n0 + TE_OUT, N); ++n) {
+    const float acc = wave_dot<WT>(x, w + (int64_t)n * freq, freq, lane);
+    if (lane == 0) silu_out[n] = silu_f32(acc + (bias ? load1_f32<WT>(bias, n) : 0.f));
+  }
 }
 
 bool aligned_rows16(const void* p, int64_t ld, int elem) {
@@ -852,13 +892,61 @@ extern "C" int srdit_gemv_f32(const float* x, int64_t ldx, const void* w, int64_
   const dim3 grid((unsigned)((N + 3) / 4), (unsigned)M);
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (w_dtype == SRDIT_DTYPE_FP32)
-    gemv_f32_kernel<float><<<grid, 256, 0, s>>>(x, ldx, static_cast<const float*>(w), ldw,
-                                                static_cast<const float*>(bias), out, ldo, (int)N,
-                                                (int)K);
+    gemv_f32_kernel<float, false><<<grid, 256, 0, s>>>(x, ldx, static_cast<const float*>(w), ldw,
+                                                       static_cast<const float*>(bias), out, ldo,
+                                                       (int)N, (int)K, nullptr);
   else
-    gemv_f32_kernel<uint16_t><<<grid, 256, 0, s>>>(x, ldx, static_cast<const uint16_t*>(w), ldw,
-                                                   static_cast<const uint16_t*>(bias), out, ldo,
-                                                   (int)N, (int)K);
+    gemv_f32_kernel<uint16_t, false><<<grid, 256, 0, s>>>(
+        x, ldx, static_cast<const uint16_t*>(w), ldw, static_cast<const uint16_t*>(bias), out, ldo,
+        (int)N, (int)K, nullptr);
   SRDIT_LAUNCH_CHECK("gemv_f32_kernel");
+  return SRDIT_OK;
+}
+
+namespace srdit {
+namespace {
+template <typename WT>
+void launch_time_embed(const float* t, int64_t freq, const void* w0, const void* b0, const void* w2,
+                       const void* b2, const void* wp, const void* bp, float* hidden, float* e,
+                       float* e0, int64_t dim, int64_t n_out, hipStream_t s) {
+  const int per = 4 * TE_OUT;
+  float* h2 = hidden + dim;
+  time_sinusoid_gemv_kernel<WT><<<(unsigned)((dim + per - 1) / per), 256, 0, s>>>(
+      t, (int)freq, static_cast<const WT*>(w0), static_cast<const WT*>(b0), hidden, (int)dim);
+  gemv_f32_kernel<WT, true><<<(unsigned)((dim + 3) / 4), 256, 0, s>>>(
+      hidden, dim, static_cast<const WT*>(w2), dim, static_cast<const WT*>(b2), e, dim, (int)dim,
+      (int)dim, h2);
+  gemv_f32_kernel<WT, false><<<(unsigned)((n_out + 3) / 4), 256, 0, s>>>(
+      h2, dim, static_cast<const WT*>(wp), dim, static_cast<const WT*>(bp), e0, n_out, (int)n_out,
+      (int)dim, nullptr);
+}
+}  // namespace
+}  // namespace srdit
+
+extern "C" int srdit_time_embed(const float* t, int64_t freq, const void* w0,
+                                const void* b0, const void* w2, const void* b2, const void* wp,
+                                const void* bp, int w_dtype, float* hidden, float* e, float* e0,
+                                int64_t dim, int64_t n_out, void* stream) {
+  const char* fn = "srdit_time_embed";
+  SRDIT_REQUIRE(t && w0 && w2 && wp && hidden && e && e0, "%s: null operand", fn);
+  SRDIT_REQUIRE(w_dtype == SRDIT_DTYPE_BF16 || w_dtype == SRDIT_DTYPE_FP32,
+                "%s: w_dtype %d is not bf16 (0) or fp32 (2)", fn, w_dtype);
+  SRDIT_REQUIRE(freq > 0 && freq % 8 == 0 && freq <= TE_MAX_FREQ && dim > 0 && dim % 8 == 0 &&
+                    n_out > 0 && dim < (1LL << 31) && n_out < (1LL << 31),
+                "%s: freq=%lld (at most %d) and dim=%lld must be positive multiples of 8, n_out=%lld "
+                "positive", fn, (long long)freq, TE_MAX_FREQ, (long long)dim, (long long)n_out);
+  const uintptr_t bmask = w_dtype == SRDIT_DTYPE_FP32 ? 3 : 1;
+  SRDIT_REQUIRE(aligned16(w0) && aligned16(w2) && aligned16(wp) && aligned16(hidden) &&
+                    (reinterpret_cast<uintptr_t>(t) & 3) == 0 &&
+                    ((reinterpret_cast<uintptr_t>(b0) | reinterpret_cast<uintptr_t>(b2) |
+                      reinterpret_cast<uintptr_t>(bp)) & bmask) == 0 &&
+                    ((reinterpret_cast<uintptr_t>(e) | reinterpret_cast<uintptr_t>(e0)) & 3) == 0,
+                "%s: weights and hidden must be 16-byte aligned, the rest to their elements", fn);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  if (w_dtype == SRDIT_DTYPE_FP32)
+    launch_time_embed<float>(t, freq, w0, b0, w2, b2, wp, bp, hidden, e, e0, dim, n_out, s);
+  else
+    launch_time_embed<uint16_t>(t, freq, w0, b0, w2, b2, wp, bp, hidden, e, e0, dim, n_out, s);
+  SRDIT_LAUNCH_CHECK("time embedding");
   return SRDIT_OK;
 }

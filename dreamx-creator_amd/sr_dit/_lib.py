@@ -73,6 +73,8 @@ SIGNATURES = {
                                    _c_i64, _c_i64, _c_int, _c_p]),
     "srdit_linear_f32_modulated": (_c_int, [_c_p, _c_i64, _c_p, _c_p, _c_p, _c_i64, _c_p, _c_int,
                                             _c_p, _c_i64, _c_i64, _c_i64, _c_i64, _c_p]),
+    "srdit_time_embed": (_c_int, [_c_p, _c_i64, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_int, _c_p,
+                                  _c_p, _c_p, _c_i64, _c_i64, _c_p]),
     "srdit_head_linear": (_c_int, [_c_p, _c_i64, _c_p, _c_int, _c_p, _c_p, _c_i64, _c_p, _c_p,
                                    _c_i64, _c_i64, _c_i64, _c_i64, _c_p]),
     "srdit_gemv_f32": (_c_int, [_c_p, _c_i64, _c_p, _c_i64, _c_p, _c_int, _c_p, _c_i64, _c_i64,
@@ -587,3 +589,40 @@ def gemv_f32(x, w, bias, out):
                                _DENSE_W_CODES[w.dtype], _ptr(out), out.stride(0), M, N, K,
                                _stream(x.device))
     _check(rc, "srdit_gemv_f32")
+
+
+def time_embed_fits(t, lins):
+    """Whether ``time_embed`` takes this timestep and these three Linears (the time
+    MLP's two and the projection)."""
+    if t.dtype != torch.float32 or t.numel() != 1 or not t.is_cuda:
+        return False
+    dt, dim = lins[0].weight.dtype, lins[0].out_features
+    if dt not in _DENSE_W_CODES or lins[0].in_features % 8 or lins[0].in_features > 2048 \
+            or dim % 8 or lins[1].in_features != dim or lins[1].out_features != dim \
+            or lins[2].in_features != dim:
+        return False
+    for m in lins:
+        w, b = m.weight, m.bias
+        if w.dtype != dt or w.device != t.device or not w.is_contiguous() or w.data_ptr() % 16:
+            return False
+        if b is not None and (b.dtype != dt or b.device != t.device or not b.is_contiguous()):
+            return False
+    return True
+
+
+def time_embed(t, lins):
+    """(e [1, dim], e0 [1, n]) fp32: the time MLP and its projection on the sinusoid of
+    the timestep t (fp32 [1]), in three launches; ``lins`` as ``time_embed_fits`` takes
+    them."""
+    l0, l2, lp = lins
+    dim, n = l0.out_features, lp.out_features
+    dev = t.device
+    hidden = torch.empty(2 * dim, dtype=torch.float32, device=dev)
+    e = torch.empty(1, dim, dtype=torch.float32, device=dev)
+    e0 = torch.empty(1, n, dtype=torch.float32, device=dev)
+    rc = load().srdit_time_embed(_ptr(t), l0.in_features, _ptr(l0.weight), _ptr(l0.bias),
+                                 _ptr(l2.weight), _ptr(l2.bias), _ptr(lp.weight), _ptr(lp.bias),
+                                 _DENSE_W_CODES[l0.weight.dtype], _ptr(hidden), _ptr(e), _ptr(e0),
+                                 dim, n, _stream(dev))
+    _check(rc, "srdit_time_embed")
+    return e, e0

@@ -721,6 +721,10 @@ class SRDiT(nn.Module):
             return out
 
         te, tp = self.time_embedding, self.time_projection
+        lins = (te[0], te[2], tp[1])
+        if _lib.time_embed_fits(t, lins):  # the whole chain in three launches, the same sums
+            e, e0 = _lib.time_embed(t, lins)
+            return e, e0.unflatten(1, (6, self.cfg.dim))
         e = lin(te[2], F.silu(lin(te[0], sinusoidal_embedding_1d(self.cfg.freq_dim, t).float())))
         e0 = lin(tp[1], F.silu(e)).unflatten(1, (6, self.cfg.dim))
         return e, e0

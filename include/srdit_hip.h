@@ -425,6 +425,20 @@ int srdit_gemv_f32(const float* x, int64_t ldx, const void* w, int64_t ldw, cons
                    int w_dtype, float* out, int64_t ldo, int64_t M, int64_t N, int64_t K,
                    void* stream);
 
+/*
+ * The time MLP and projection on one timestep in three launches: x = the
+ * sinusoid of t (fp32 [1]; cos then sin of t 10000^(-i / (freq / 2)), formed in
+ * 64 bits, rounded to fp32), e [dim] = silu(x w0^T + b0) w2^T + b2 and e0 [n_out] =
+ * silu(e) wp^T + bp, fp32, each sum as srdit_gemv_f32 takes it.  w0 [dim, freq],
+ * w2 [dim, dim], wp [n_out, dim] contiguous and 16-byte aligned, all bf16 or all
+ * fp32 (w_dtype) with their biases (which may be NULL); hidden: fp32 [2 dim]
+ * scratch, 16-byte aligned; freq and dim multiples of 8, freq <= 2048.  Replaces
+ * models.py:1845-1849 and :67-77.
+ */
+int srdit_time_embed(const float* t, int64_t freq, const void* w0, const void* b0, const void* w2,
+                     const void* b2, const void* wp, const void* bp, int w_dtype, float* hidden,
+                     float* e, float* e0, int64_t dim, int64_t n_out, void* stream);
+
 /* Message of the last failed call on this thread (NUL-terminated, truncated to
  * len).  Returns the message length. */
 int srdit_last_error(char* buf, int len);
