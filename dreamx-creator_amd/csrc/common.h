@@ -60,13 +60,21 @@ typedef int i32x4_t __attribute__((__vector_size__(4 * sizeof(int))));
 typedef int i32x2_t __attribute__((__vector_size__(2 * sizeof(int))));
 
 // GELU with the tanh approximation, as torch evaluates it in fp32:
-// 0.5 x (1 + tanh(sqrt(2/pi) (x + 0.044715 x^3))).
+// 0.5 x (1 + tanh(sqrt(2/pi) (x + 0.044715 x^3))).  The tanh is
+// 1 - 2 / (e^{2|u|} + 1) with u's sign, on the hardware exponential and
+// reciprocal (an ulp each): for large |u| the quotient is small, so its error is
+// far below tanh's last place and 1 + tanh cancels to the same multiple of 2^-24;
+// near 0 the error is one 2^-24, which 1 + tanh absorbs.  (The library's tanhf, with
+// its two branches and its division, took 170 us of the 567 us of a 10800 x 14336 x
+// 3072 GEMM with this epilogue.)
 __device__ __forceinline__ float gelu_tanh(float x) {
   const float kBeta = 0.7978845608028654f;  // sqrt(2 / pi)
   const float kKappa = 0.044715f;
   const float x3 = x * x * x;
   const float inner = kBeta * (x + kKappa * x3);
-  return 0.5f * x * (1.0f + tanhf(inner));
+  const float ex = __builtin_amdgcn_exp2f(__builtin_fabsf(inner) * 2.8853900817779268f);  // 2 log2 e
+  const float th = __builtin_fmaf(-2.0f, __builtin_amdgcn_rcpf(ex + 1.0f), 1.0f);
+  return 0.5f * x * (1.0f + __builtin_copysignf(th, inner));
 }
 
 // bf16 round trip (nearest even): the value torch holds after .to(bf16).
