@@ -566,8 +566,11 @@ void window_group_kernel(GroupArgs a) {
   // Slots this wavefront computes: the member's, less (AMODE 1) the anchor
   // frames none of its valid queries is admitted to.  Such a slot would add
   // exp2(-inf) = 0 to every row, so its softmax, P.V and S^T MFMAs are
-  // skipped; the fills go on (both wavefronts share them).
-  uint32_t wact = act;
+  // skipped; the fills go on (both wavefronts share them).  A wavefront without
+  // any valid query (the second half of a ragged edge window's tile) computes
+  // nothing (34 x 60 tokens, 8 x 8 blocks: 12 of 40 windows; 253.0 -> 247.7 us, the
+  // same process; 45 x 80 tokens: 391 us either way).
+  uint32_t wact = __any(qvalid) ? act : 0u;
   if constexpr (AMODE == 1) {
     for (int k = 0; k < n_anc; ++k) {
       const int fs_ = P + nsh + k;
