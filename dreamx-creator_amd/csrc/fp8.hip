@@ -198,27 +198,60 @@ __global__ __launch_bounds__(256) void quant_rowwise_long_kernel(const T* __rest
 
 __global__ void clear_u32_kernel(uint32_t* p) { *p = 0u; }
 
-// Grid-stride amax: each wavefront walks rows wave_id, wave_id + n_waves, ...
-template <typename T>
+// The per-tensor passes walk contiguous tensors as one array of 8-element chunks
+// (FLAT; every workgroup takes the same share, FQ chunks per lane in flight) and
+// strided ones row by row, a wavefront per row.
+constexpr int FQ = 8;              // chunks per lane in flight
+constexpr unsigned FLAT_WGS = 1024;  // workgroups of a flat walk: four per CU
+
+template <typename T, typename F>
+__device__ __forceinline__ void flat_walk(const T* __restrict__ x, int64_t n, F&& use) {
+  const int64_t step = (int64_t)gridDim.x * 256 * FQ;
+  for (int64_t base = (int64_t)blockIdx.x * 256 * FQ + threadIdx.x; base < n; base += step) {
+    Raw8<T> v[FQ];
+#pragma unroll
+    for (int u = 0; u < FQ; ++u) {
+      const int64_t c = base + 256 * u;
+      if (c < n) v[u].load(x, c);
+      else v[u].clear();
+    }
+#pragma unroll
+    for (int u = 0; u < FQ; ++u) {
+      float f[8];
+      v[u].get(f);
+      use(base + 256 * u, f);
+    }
+  }
+}
+
+// Max |x| into *amax_ws.  Each workgroup reads the word once (raise_max_word), and
+// those reads meet in one memory channel, so there are few workgroups: 21600 x 3072
+// took 39.6 us with 4096 workgroups of one row per wavefront (some two, most one),
+// 27.0 us with 1024 equal shares.
+template <typename T, bool FLAT>
 __global__ __launch_bounds__(256) void amax_kernel(const T* __restrict__ x, int64_t M, int64_t K,
                                                    int64_t ldx, uint32_t* __restrict__ amax_ws) {
   __shared__ uint32_t part[4];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int64_t nchunk = K >> 3;
   uint32_t amax = 0;
-  for (int64_t row = (int64_t)blockIdx.x * 4 + wave; row < M; row += (int64_t)gridDim.x * 4) {
-    const T* xr = x + row * ldx;
-    // four chunks per lane in flight; a clamped index re-reads a chunk already
-    // counted, which leaves the max unchanged
-    for (int64_t c0 = lane; c0 < nchunk; c0 += 256) {
-      float f[4][8];
+  if constexpr (FLAT) {
+    flat_walk<T>(x, M * nchunk, [&](int64_t, const float f[8]) { amax = abs_bits_max8(f, amax); });
+  } else {
+    for (int64_t row = (int64_t)blockIdx.x * 4 + wave; row < M; row += (int64_t)gridDim.x * 4) {
+      const T* xr = x + row * ldx;
+      // four chunks per lane in flight; a clamped index re-reads a chunk already
+      // counted, which leaves the max unchanged
+      for (int64_t c0 = lane; c0 < nchunk; c0 += 256) {
+        float f[4][8];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int64_t c = c0 + 64 * u;
-        Load8<T>::get(xr, c < nchunk ? c : nchunk - 1, f[u]);
+        for (int u = 0; u < 4; ++u) {
+          const int64_t c = c0 + 64 * u;
+          Load8<T>::get(xr, c < nchunk ? c : nchunk - 1, f[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) amax = abs_bits_max8(f[u], amax);
       }
-#pragma unroll
-      for (int u = 0; u < 4; ++u) amax = abs_bits_max8(f[u], amax);
     }
   }
   amax = wave_umax(amax);
@@ -230,9 +263,9 @@ __global__ __launch_bounds__(256) void amax_kernel(const T* __restrict__ x, int6
   }
 }
 
-constexpr int QU = 4;  // 16-byte chunks per lane in flight in the quantise pass
+constexpr int QU = 4;  // 16-byte chunks per lane in flight in the row-by-row passes
 
-template <typename T>
+template <typename T, bool FLAT>
 __global__ __launch_bounds__(256) void quant_tensor_kernel(const T* __restrict__ x, int64_t M,
                                                            int64_t K, int64_t ldx,
                                                            uint8_t* __restrict__ xq,
@@ -243,6 +276,15 @@ __global__ __launch_bounds__(256) void quant_tensor_kernel(const T* __restrict__
   const SharedDivisor sd(s);
   if (blockIdx.x == 0 && threadIdx.x == 0) scale[0] = s;
   const int64_t nchunk = K >> 3;
+  if constexpr (FLAT) {
+    uint2* q = reinterpret_cast<uint2*>(xq);
+    const int64_t n = M * nchunk;
+    if (sd.fast)
+      flat_walk<T>(x, n, [&](int64_t c, const float f[8]) { if (c < n) q[c] = to_e4m3x8<true>(f, sd); });
+    else
+      flat_walk<T>(x, n, [&](int64_t c, const float f[8]) { if (c < n) q[c] = to_e4m3x8(f, sd); });
+    return;
+  }
   for (int64_t row = (int64_t)blockIdx.x * 4 + wave; row < M; row += (int64_t)gridDim.x * 4) {
     const T* xr = x + row * ldx;
     uint2* qr = reinterpret_cast<uint2*>(xq + row * K);
@@ -261,6 +303,35 @@ __global__ __launch_bounds__(256) void quant_tensor_kernel(const T* __restrict__
         if (c < nchunk) qr[c] = to_e4m3x8(f[u], sd);
       }
     }
+  }
+}
+
+template <typename T>
+void launch_amax(const void* x, int64_t M, int64_t K, int64_t ldx, uint32_t* amax_ws,
+                 hipStream_t s) {
+  const T* xp = static_cast<const T*>(x);
+  if (ldx == K || M == 1) {
+    const int64_t wgs = (M * (K >> 3) + 256 * FQ - 1) / (256 * FQ);
+    amax_kernel<T, true><<<(unsigned)(wgs < FLAT_WGS ? wgs : FLAT_WGS), 256, 0, s>>>(xp, M, K, ldx, amax_ws);
+  } else {
+    const int64_t rows4 = (M + 3) / 4;
+    amax_kernel<T, false><<<(unsigned)(rows4 < 4096 ? rows4 : 4096), 256, 0, s>>>(xp, M, K, ldx, amax_ws);
+  }
+}
+
+template <typename T>
+void launch_quant_tensor(const void* x, int64_t M, int64_t K, int64_t ldx, void* xq, float* scale,
+                         const uint32_t* amax_ws, hipStream_t s) {
+  const T* xp = static_cast<const T*>(x);
+  uint8_t* qp = static_cast<uint8_t*>(xq);
+  if (ldx == K || M == 1) {
+    const int64_t wgs = (M * (K >> 3) + 256 * FQ - 1) / (256 * FQ);
+    quant_tensor_kernel<T, true><<<(unsigned)(wgs < FLAT_WGS ? wgs : FLAT_WGS), 256, 0, s>>>(
+        xp, M, K, ldx, qp, scale, amax_ws);
+  } else {
+    const int64_t rows4 = (M + 3) / 4;
+    quant_tensor_kernel<T, false><<<(unsigned)(rows4 < 4096 ? rows4 : 4096), 256, 0, s>>>(
+        xp, M, K, ldx, qp, scale, amax_ws);
   }
 }
 
@@ -1221,14 +1292,11 @@ extern "C" int srdit_fp8_quant_tensor(const void* x, int64_t M, int64_t K, int64
   hipStream_t s = static_cast<hipStream_t>(stream);
   return dispatch_quant_dtype(dtype, [&](auto tag) -> int {
     using T = std::remove_const_t<std::remove_pointer_t<decltype(tag)>>;
-    const int64_t rows4 = (M + 3) / 4;
-    const unsigned blocks = (unsigned)(rows4 < 4096 ? rows4 : 4096);
     clear_u32_kernel<<<1, 1, 0, s>>>(amax_ws);
     SRDIT_LAUNCH_CHECK("clear_u32_kernel");
-    amax_kernel<T><<<blocks, 256, 0, s>>>(static_cast<const T*>(x), M, K, ldx, amax_ws);
+    launch_amax<T>(x, M, K, ldx, amax_ws, s);
     SRDIT_LAUNCH_CHECK("amax_kernel");
-    quant_tensor_kernel<T><<<blocks, 256, 0, s>>>(static_cast<const T*>(x), M, K, ldx,
-                                                  static_cast<uint8_t*>(xq), scale, amax_ws);
+    launch_quant_tensor<T>(x, M, K, ldx, xq, scale, amax_ws, s);
     SRDIT_LAUNCH_CHECK("quant_tensor_kernel");
     return SRDIT_OK;
   });
@@ -1510,10 +1578,7 @@ extern "C" int srdit_fp8_quant_apply(const void* x, int64_t M, int64_t K, int64_
   hipStream_t s = static_cast<hipStream_t>(stream);
   return dispatch_quant_dtype(dtype, [&](auto tag) -> int {
     using T = std::remove_const_t<std::remove_pointer_t<decltype(tag)>>;
-    const int64_t rows4 = (M + 3) / 4;
-    const unsigned blocks = (unsigned)(rows4 < 4096 ? rows4 : 4096);
-    quant_tensor_kernel<T><<<blocks, 256, 0, s>>>(static_cast<const T*>(x), M, K, ldx,
-                                                  static_cast<uint8_t*>(xq), scale, amax_ws);
+    launch_quant_tensor<T>(x, M, K, ldx, xq, scale, amax_ws, s);
     SRDIT_LAUNCH_CHECK("quant_tensor_kernel");
     return SRDIT_OK;
   });
@@ -1661,14 +1726,11 @@ extern "C" int srdit_fp8_linear_tensor_static(const void* x, int64_t M, int64_t 
   hipStream_t s = static_cast<hipStream_t>(stream);
   int rc = dispatch_quant_dtype(dtype, [&](auto tag) -> int {
     using T = std::remove_const_t<std::remove_pointer_t<decltype(tag)>>;
-    const int64_t rows4 = (M + 3) / 4;
-    const unsigned blocks = (unsigned)(rows4 < 4096 ? rows4 : 4096);
     clear_u32_kernel<<<1, 1, 0, s>>>(amax);
     SRDIT_LAUNCH_CHECK("clear_u32_kernel");
-    amax_kernel<T><<<blocks, 256, 0, s>>>(static_cast<const T*>(x), M, K, ldx, amax);
+    launch_amax<T>(x, M, K, ldx, amax, s);
     SRDIT_LAUNCH_CHECK("amax_kernel");
-    quant_tensor_kernel<T><<<blocks, 256, 0, s>>>(static_cast<const T*>(x), M, K, ldx, codes,
-                                                  scale, amax);
+    launch_quant_tensor<T>(x, M, K, ldx, codes, scale, amax, s);
     SRDIT_LAUNCH_CHECK("quant_tensor_kernel");
     return SRDIT_OK;
   });
