@@ -67,6 +67,8 @@ SIGNATURES = {
     "srdit_residual_ln_modulate": (_c_int, [_c_p, _c_p, _c_p, _c_i64, _c_int, _c_i64, _c_i64,
                                             _c_p, _c_i64, _c_p, _c_p, _c_p, _c_p, _c_f, _c_p,
                                             _c_i64, _c_p, _c_p]),
+    "srdit_residual_ln_quant": (_c_int, [_c_p, _c_p, _c_p, _c_i64, _c_int, _c_i64, _c_i64, _c_p,
+                                         _c_i64, _c_p, _c_p, _c_p, _c_p, _c_f, _c_p, _c_p, _c_p]),
     "srdit_rmsnorm_rope": (_c_int, [_c_p, _c_i64, _c_int, _c_i64, _c_p, _c_f, _c_p, _c_int, _c_p,
                                     _c_p]),
     "srdit_bf16_linear": (_c_int, [_c_p, _c_i64, _c_p, _c_i64, _c_p, _c_p, _c_i64, _c_i64,
@@ -470,6 +472,28 @@ def residual_ln_modulate(x, y, gate, x_out, ln_w, ln_b, scale, shift, eps, out, 
         x_out.stride(0), _ptr(ln_w), _ptr(ln_b), _ptr(scale), _ptr(shift), float(eps), _ptr(out),
         out.stride(0), _ptr(amax_ws), _stream(x.device))
     _check(rc, "srdit_residual_ln_modulate")
+
+
+def residual_ln_quant(x, y, gate, x_out, ln_w, ln_b, scale, shift, eps, xq, xs):
+    """x_out = bf16(x + y * gate) (y, gate and x_out may be None: x as it is), and the
+    row-wise e4m3 codes xq [M, K] and scales xs [M] of its LayerNorm and modulation, in
+    one pass: the same bits as residual_ln_modulate followed by fp8_quant_rowwise."""
+    _bf16_rows("residual_ln_quant x", x)
+    for nm, t in (("y", y), ("x_out", x_out)):
+        if t is not None:
+            _bf16_rows(f"residual_ln_quant {nm}", t)
+            if t.shape != x.shape:
+                raise ValueError(f"residual_ln_quant: {nm} {tuple(t.shape)} is not {tuple(x.shape)}")
+    M, K = x.shape
+    if xq.dtype != torch.float8_e4m3fn or tuple(xq.shape) != (M, K) or not xq.is_contiguous():
+        raise ValueError(f"residual_ln_quant: xq must be contiguous float8_e4m3fn [{M}, {K}]")
+    if xs.dtype != torch.float32 or xs.numel() != M or not xs.is_contiguous():
+        raise ValueError(f"residual_ln_quant: xs must be contiguous float32 [{M}]")
+    rc = load().srdit_residual_ln_quant(
+        _ptr(x), _ptr(y), _ptr(gate), M, K, x.stride(0), 0 if y is None else y.stride(0),
+        _ptr(x_out), 0 if x_out is None else x_out.stride(0), _ptr(ln_w), _ptr(ln_b), _ptr(scale),
+        _ptr(shift), float(eps), _ptr(xq), _ptr(xs), _stream(x.device))
+    _check(rc, "srdit_residual_ln_quant")
 
 
 def rmsnorm_rope(x, w, eps, rope_cs, head_dim, out):

@@ -423,16 +423,29 @@ class Block(nn.Module):
                 _lib.fp8_quant_apply(t, tq, ts, word)
             return tq, ts
 
+        def norm_quant(x, res, norm, sc, sh):
+            """The residual stream with ``res = (y, gate)`` applied (or x itself) and
+            the codes and scale of its LayerNorm, modulated by sc and sh.  Row-wise
+            codes leave the LayerNorm's own pass, whose row sits in registers (up to
+            4096 wide); the per-tensor scale needs every row's amax first."""
+            xr = x if res is None else torch.empty_like(x)
+            if rowwise and dim <= 4096:
+                tq = torch.empty(s, dim, dtype=FP8_DTYPE, device=dev)
+                ts = torch.empty(s, dtype=torch.float32, device=dev)
+                y, gate = (None, None) if res is None else res
+                _lib.residual_ln_quant(x, y, gate, None if res is None else xr, norm.weight,
+                                       norm.bias, sc, sh, norm.eps, tq, ts)
+                return xr, tq, ts
+            t = torch.empty(s, dim, dtype=bf, device=dev)
+            if res is None:
+                _lib.ln_modulate(x, norm.weight, norm.bias, sc, sh, norm.eps, t, a0)
+            else:
+                _lib.residual_ln_modulate(x, res[0], res[1], xr, norm.weight, norm.bias, sc, sh,
+                                          norm.eps, t, a0)
+            return (xr, *quant_from(t, a0))
+
         # self-attention
-        attn_in = torch.empty(s, dim, dtype=bf, device=dev)
-        if pending is None:
-            _lib.ln_modulate(x, None, None, mod[1], mod[0], self.norm1.eps, attn_in, a0)
-        else:
-            xr = torch.empty_like(x)
-            _lib.residual_ln_modulate(x, pending[0], pending[1], xr, None, None, mod[1], mod[0],
-                                      self.norm1.eps, attn_in, a0)
-            x = xr
-        xq, xs = quant_from(attn_in, a0)
+        x, xq, xs = norm_quant(x, pending, self.norm1, mod[1], mod[0])
         pack = self._qkv_pack() if (QKV_PACK and not kv_only and dim % 256 == 0) else None
         if pack is not None:
             # q, k and v from one GEMM over xq; V is then copied to its ring region
@@ -489,10 +502,7 @@ class Block(nn.Module):
         y = sa.o.gemm(*quant_from(att_out.view(s, dim), a2))
 
         # gated residual and norm3, then the cross-attention
-        x1, xn = torch.empty_like(x), torch.empty_like(x)
-        _lib.residual_ln_modulate(x, y, mod[2], x1, self.norm3.weight, self.norm3.bias, None, None,
-                                  self.norm3.eps, xn, a0)
-        xq, xs = quant_from(xn, a0)
+        x1, xq, xs = norm_quant(x, (y, mod[2]), self.norm3, None, None)
         cq = torch.empty(s, dim, dtype=bf, device=dev)
         _lib.rmsnorm_rope(ca.q.gemm(xq, xs), ca.norm_q.weight, ca.norm_q.eps, None, d, cq)
         lc = context.shape[0]
@@ -503,10 +513,7 @@ class Block(nn.Module):
         co = ca.o.gemm(*quant_from(c_out.view(s, dim), a2))
 
         # residual, norm2 and modulation, then the FFN
-        x2, ffn_in = torch.empty_like(x), torch.empty_like(x)
-        _lib.residual_ln_modulate(x1, co, geom["ones"], x2, None, None, mod[4], mod[3],
-                                  self.norm2.eps, ffn_in, a0)
-        xq, xs = quant_from(ffn_in, a0)
+        x2, xq, xs = norm_quant(x1, (co, geom["ones"]), self.norm2, mod[4], mod[3])
         if rowwise:
             hq, hs = quant_from(self.ffn[0].gemm(xq, xs, epilogue=1), None)  # GELU in the epilogue
         elif FFN_GELU_IN_GEMM:

@@ -363,6 +363,17 @@ int srdit_residual_ln_modulate(const void* x, const void* y, const float* gate, 
                                uint32_t* amax_ws, void* stream);
 
 /*
+ * srdit_residual_ln_modulate with its output quantised row by row instead of
+ * stored: xq [M, K] e4m3 and xs [M] are srdit_fp8_quant_rowwise of out, bit for
+ * bit.  y, gate and x_out may all be NULL (no residual: the LayerNorm of x).
+ * K <= 4096; scale and shift 16-byte aligned.
+ */
+int srdit_residual_ln_quant(const void* x, const void* y, const float* gate, int64_t M, int K,
+                            int64_t ldx, int64_t ldy, void* x_out, int64_t ldxo, const void* ln_w,
+                            const void* ln_b, const float* scale, const float* shift, float eps,
+                            void* xq, float* xs, void* stream);
+
+/*
  * RMSNorm over each row of x [M, K] (bf16, K = heads * head_dim) with weight w
  * (bf16 [K]), then RoPE per head: pair j of a head rotated by
  * (cos, sin) = rope_cs[row][j] (fp32 pairs, [M, head_dim/2]); rope_cs NULL skips
