@@ -1541,6 +1541,17 @@ extern "C" int srdit_fp8_gemm(const void* a, const void* b, const float* sa, int
                          stream, "srdit_fp8_gemm");
 }
 
+extern "C" int srdit_fp8_linear(const void* x, int64_t M, int64_t K, int64_t ldx, int dtype,
+                                const void* w, const float* w_scale, int64_t w_scale_cols,
+                                const void* bias, void* xq, float* xs, uint32_t* amax_ws, void* out,
+                                int64_t N, int64_t ldo, int rowwise, void* stream) {
+  const int rc = rowwise ? srdit_fp8_quant_rowwise(x, M, K, ldx, dtype, xq, xs, stream)
+                         : srdit_fp8_quant_tensor(x, M, K, ldx, dtype, xq, xs, amax_ws, stream);
+  if (rc) return rc;
+  return fp8_gemm_launch(xq, w, xs, rowwise ? M : 1, w_scale, w_scale_cols, bias, out, M, N, K, ldo,
+                         0, nullptr, stream, "srdit_fp8_linear");
+}
+
 extern "C" int srdit_fp8_gemm_ex(const void* a, const void* b, const float* sa, int64_t sa_rows,
                                  const float* sb, int64_t sb_cols, const void* bias, void* out,
                                  int64_t M, int64_t N, int64_t K, int64_t ldo, int epilogue,

@@ -67,6 +67,8 @@ SIGNATURES = {
     "srdit_residual_ln_modulate": (_c_int, [_c_p, _c_p, _c_p, _c_i64, _c_int, _c_i64, _c_i64,
                                             _c_p, _c_i64, _c_p, _c_p, _c_p, _c_p, _c_f, _c_p,
                                             _c_i64, _c_p, _c_p]),
+    "srdit_fp8_linear": (_c_int, [_c_p, _c_i64, _c_i64, _c_i64, _c_int, _c_p, _c_p, _c_i64, _c_p,
+                                  _c_p, _c_p, _c_p, _c_p, _c_i64, _c_i64, _c_int, _c_p]),
     "srdit_residual_ln_quant": (_c_int, [_c_p, _c_p, _c_p, _c_i64, _c_int, _c_i64, _c_i64, _c_p,
                                          _c_i64, _c_p, _c_p, _c_p, _c_p, _c_f, _c_p, _c_p, _c_p]),
     "srdit_rmsnorm_rope": (_c_int, [_c_p, _c_i64, _c_int, _c_i64, _c_p, _c_f, _c_p, _c_int, _c_p,
@@ -124,7 +126,9 @@ def _ptr(t) -> int | None:
 
 
 def _stream(device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    # the raw handle, without a torch.cuda.Stream object around it (1.5 us a call)
+    idx = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if idx is None else idx)
 
 
 def _ex_args(ring, amax_out):
@@ -272,6 +276,38 @@ def fp8_gemm(a, b, sa, sb, bias, out):
                                int(sb.numel()), _ptr(bias), _ptr(out), M, N, K,
                                out.stride(0), _stream(a.device))
     _check(rc, "srdit_fp8_gemm")
+
+
+def fp8_linear(x, w, w_scale, bias, rowwise):
+    """bf16 [M, N] = x [M, K] quantised (per row, or per tensor) . w [N, K]^T * scales + bias:
+    fp8_quant_rowwise or fp8_quant_tensor, then fp8_gemm, as one call.  x: contiguous,
+    16-byte aligned.  The codes, scales and amax word share one scratch tensor."""
+    if x.dim() != 2 or not x.is_contiguous():
+        raise ValueError(f"fp8_linear needs a contiguous 2-D input, got shape {tuple(x.shape)} "
+                         f"strides {x.stride()}")
+    dt = QUANT_DTYPE_CODES.get(x.dtype)
+    if dt is None:
+        raise ValueError(f"fp8 quantiser input must be bf16, fp16 or fp32, got {x.dtype}")
+    M, K = x.shape
+    N = w.shape[0]
+    if w.dtype != torch.float8_e4m3fn or w.dim() != 2 or w.shape[1] != K or not w.is_contiguous():
+        raise ValueError(f"fp8_linear: w must be a contiguous float8_e4m3fn [N, {K}] tensor")
+    if w_scale.dtype != torch.float32 or not w_scale.is_contiguous():
+        raise ValueError("fp8_linear: w_scale must be contiguous float32")
+    if bias is not None and (bias.dtype != torch.bfloat16 or bias.numel() != N
+                             or not bias.is_contiguous()):
+        raise ValueError(f"fp8_linear: bias must be {N} contiguous bf16 values")
+    out = torch.empty(M, N, dtype=torch.bfloat16, device=x.device)
+    codes = (M * K + 15) & -16                       # then the scales, then the amax word
+    n_scales = M if rowwise else 1
+    scratch = torch.empty(codes + 4 * n_scales + 4, dtype=torch.uint8, device=x.device)
+    p = scratch.data_ptr()
+    rc = load().srdit_fp8_linear(x.data_ptr(), M, K, K, dt, w.data_ptr(), w_scale.data_ptr(),
+                                 w_scale.numel(), _ptr(bias), p, p + codes,
+                                 p + codes + 4 * n_scales, out.data_ptr(), N, N, int(rowwise),
+                                 _stream(x.device))
+    _check(rc, "srdit_fp8_linear")
+    return out
 
 
 #: epilogue flag of srdit_fp8_gemm_ex kept for old callers; it has no effect

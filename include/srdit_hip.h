@@ -280,6 +280,16 @@ int srdit_fp8_quant_tensor_gelu_ex(const void* x, int64_t M, int64_t K, int64_t 
  * Every GEMM runs on that kernel now; the flag is accepted and has no effect. */
 #define SRDIT_GEMM_MFMA 0x100
 
+/*
+ * The fp8 Linear as Fp8Linear.forward runs it (fp8_linear.py:282-297) in one call:
+ * srdit_fp8_quant_rowwise (rowwise != 0) or srdit_fp8_quant_tensor of x [M, K] into
+ * xq and xs (M scales, or 1 with amax_ws), then srdit_fp8_gemm with w [N, K] e4m3.
+ */
+int srdit_fp8_linear(const void* x, int64_t M, int64_t K, int64_t ldx, int dtype, const void* w,
+                     const float* w_scale, int64_t w_scale_cols, const void* bias, void* xq,
+                     float* xs, uint32_t* amax_ws, void* out, int64_t N, int64_t ldo, int rowwise,
+                     void* stream);
+
 /* Flag for the epilogue argument of srdit_fp8_gemm_ex (epilogue 0 only):
  * amax_out receives the largest positive output instead of max |out| (the
  * float bits of a non-negative value, 0 when every output is negative, the
