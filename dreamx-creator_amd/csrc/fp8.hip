@@ -1037,16 +1037,24 @@ void fp8_gemm_kernel(const MatmulArgs g) {
 // 512 rows 31.7 -> 10.0, 1024 rows 32.8 -> 17.3, 2048 rows 33.6 -> 29.3; bf16
 // operands against the register-fed kernel of dense.hip, 512 x 3072: K = 4096
 // 80.5 -> 24.7 us, K = 3072 63.6 -> 20.4 us.
+//
+// KG = 2 (bf16): two groups of four wavefronts take alternate K stages of the tile
+// through rings of their own, and the second group's sums are added to the first's,
+// so a CU that holds one workgroup has two wavefronts per SIMD.  The order of the K
+// sum then differs from the large kernel's.  Measured, bf16, KG 1 -> 2: 256 x 3072 x
+// 4096 18.3 -> 15.0 us (MI = 1), 512 x 3072 x 4096 23.6 (MI = 1) -> 21.6 (MI = 2).
 constexpr int GS_NST = 3;
 
-template <int EPI, int AMAX, int BF, int MI>
-__global__ __launch_bounds__(256) void small_tile_matmul_kernel(const MatmulArgs g) {
+template <int EPI, int AMAX, int BF, int MI, int KG = 1>
+__global__ __launch_bounds__(256 * KG) void small_tile_matmul_kernel(const MatmulArgs g) {
   constexpr int TM = 64 * MI, TN = 64, NST = GS_NST;
   constexpr int STAGE = (TM + TN) * G_FK;
   constexpr int FILLS = 2 * MI + 2;  // fill DMAs per wavefront per stage
-  __shared__ __attribute__((aligned(1024))) uint8_t smem[NST * STAGE];
+  __shared__ __attribute__((aligned(1024))) uint8_t smem_all[KG * NST * STAGE];
   const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wave_wg = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wave = wave_wg & 3, kg = KG == 1 ? 0 : wave_wg >> 2;  // kg: the group's K share
+  uint8_t* const smem = smem_all + kg * (NST * STAGE);
   const int wm = wave & 1, wn = wave >> 1;
   const uint32_t tiles_m = (uint32_t)(g.M + TM - 1) / TM;
   const uint32_t task = xcd_task(blockIdx.x, gridDim.x);
@@ -1074,7 +1082,7 @@ __global__ __launch_bounds__(256) void small_tile_matmul_kernel(const MatmulArgs
   const int brow = (wave * 16 + (lane >> 3)) * g.K;
   auto fill = [&](int s, int slot) __attribute__((always_inline)) {
     const uint32_t base = lds_base + slot * STAGE;
-    const int koff = s * G_FK;
+    const int koff = (s * KG + kg) * G_FK;
 #pragma unroll
     for (int q = 0; q < 2 * MI; ++q)
       dma(ra, arow + q * 8 * g.K + ((q & 1) ? sw_odd : sw_even), koff,
@@ -1130,7 +1138,7 @@ __global__ __launch_bounds__(256) void small_tile_matmul_kernel(const MatmulArgs
   };
   using K0 = std::integral_constant<int, 0>;
   using K1 = std::integral_constant<int, 1>;
-  const int nks = g.K / G_FK;
+  const int nks = g.K / G_FK / KG;  // stages of this group (the host: a multiple of KG)
 #pragma unroll
   for (int s = 0; s < NST; ++s)
     if (s < nks) fill(s, s);
@@ -1166,6 +1174,28 @@ __global__ __launch_bounds__(256) void small_tile_matmul_kernel(const MatmulArgs
   waitcnt_vm<0>();
   __builtin_amdgcn_s_barrier();
   compiler_fence_gemm();
+  if constexpr (KG == 2) {  // the second group's sums join the first's
+    // past the transposes' 8 KB
+    f32x4_t* part = reinterpret_cast<f32x4_t*>(smem_all + 8192) + (wave * MI * 4) * 64 + lane;
+    if (kg == 1) {
+#pragma unroll
+      for (int j = 0; j < MI; ++j)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          part[(j * 4 + q) * 64] =
+              f32x4_t{acc[j][4 * q], acc[j][4 * q + 1], acc[j][4 * q + 2], acc[j][4 * q + 3]};
+    }
+    __syncthreads();
+    if (kg == 1) return;  // no barrier follows
+#pragma unroll
+    for (int j = 0; j < MI; ++j)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const f32x4_t v = part[(j * 4 + q) * 64];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[j][4 * q + r] += v[r];
+      }
+  }
 
   const int rows = min(TM, g.M - m0);
   int64_t obase = (int64_t)m0 * g.ldo;
@@ -1366,6 +1396,18 @@ int small_tile_rows(int64_t M, int64_t N, int64_t cus) {
   return (M + 127) / 128 * tn <= 3 * cus ? 2 : 0;
 }
 
+// bf16 operands on small tiles: the rows per tile (in 64s) of two K groups, 0 for one
+// group.  Two pay while every workgroup has a CU of its own (their rings take 96 or
+// 144 KB): 512 x 1536 x 4096 (192 of 64 x 64) 17.9 -> 14.8 us, 512 x 3072 x 3072 (192 of
+// 128 x 64) 20.4 -> 18.4; past that they are slower (1024 x 3072 x 4096 34.2 -> 42.1), as
+// on few K stages (512 x 3072 x 1024, 16 stages, 7.8 -> 8.1).
+int k_group_rows(int64_t M, int64_t N, int64_t cus, int nks) {
+  if (nks % 2 != 0 || nks < 24) return 0;
+  const int64_t tn = (N + 63) / 64;
+  if ((M + 63) / 64 * tn <= cus) return 1;
+  return (M + 127) / 128 * tn <= cus ? 2 : 0;
+}
+
 // The rows to leave to small tiles when the last, partial tile row of 256 x 256
 // tiles opens a round of its own (10800 x 3072: 516 tiles, the 12 of the last
 // 48 rows in a third round of 256 CUs): that round costs a whole tile's K loop
@@ -1468,6 +1510,19 @@ int fp8_gemm_launch(const void* a, const void* b, const float* sa, int64_t sa_ro
     SRDIT_LAUNCH_CHECK("small_tile_matmul_kernel");
     return SRDIT_OK;
   };
+  const int kg_rows = bf16 ? k_group_rows(M, N, cus, g.K / G_FK) : 0;
+  if (kg_rows) {
+    auto launch_kg = [&](auto mi_c) -> int {
+      constexpr int MI = decltype(mi_c)::value;
+      const unsigned nwg = (unsigned)((M + 64 * MI - 1) / (64 * MI) * ((N + 63) / 64));
+      if (epilogue == 0) small_tile_matmul_kernel<0, 0, 1, MI, 2><<<nwg, 512, 0, s>>>(g);
+      else small_tile_matmul_kernel<1, 0, 1, MI, 2><<<nwg, 512, 0, s>>>(g);
+      SRDIT_LAUNCH_CHECK("small_tile_matmul_kernel (two K groups)");
+      return SRDIT_OK;
+    };
+    return kg_rows == 1 ? launch_kg(std::integral_constant<int, 1>{})
+                        : launch_kg(std::integral_constant<int, 2>{});
+  }
   const int mi = small_tile_rows(M, N, cus);
   if (mi == 1) return launch_small(g, std::integral_constant<int, 1>{});
   if (mi == 2) return launch_small(g, std::integral_constant<int, 2>{});

@@ -89,7 +89,11 @@ def test_small_tiles_split_output():
 
 @pytest.mark.parametrize("M,N,K,gelu", [(1, 16, 64, False), (512, 3072, 4096, True),
                                         (65, 1536, 192, False), (1000, 3072, 128, True),
-                                        (2500, 3072, 512, False)])
+                                        (2500, 3072, 512, False),
+                                        # two K groups: 24 and 26 stages, 64- and 128-row
+                                        # tiles, ragged rows and columns; 25 stages: one
+                                        (1, 16, 1536, False), (130, 1040, 1664, True),
+                                        (500, 3056, 1536, True), (385, 3072, 1600, False)])
 def test_bf16_small_tiles_match_float64(M, N, K, gelu):
     """bf16 operands: the fp32 sum's K 2^-24 of the sum of |terms|, half an ulp of the
     rounding, and a full one where the GELU reads a value at a rounding boundary."""
