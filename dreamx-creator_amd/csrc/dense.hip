@@ -17,13 +17,18 @@
 // result rounds once to the output dtype, and the GELU acts on the rounded
 // bf16 value and rounds again.
 //
-// The MFMA operands are read straight from global memory (L2), without LDS
-// staging: these GEMMs are either bound by their output stores (patch
-// embedding: K = 64) or are small (text embedding: 512 rows; head: 64 output
-// columns), and one wave's 32-row operand slice is re-read by at most two
-// waves of its workgroup.  Lanes 0-31 of an MFMA operand hold rows 0-31 of
-// k-slice [k0, k0+8), lanes 32-63 the same rows at [k0+8, k0+16): a k index is
-// paired the same way in A and W, so the sum over k is the GEMM's.
+//   head_linear   linear_f32_modulated with bf16 weights on bf16 MFMAs, s1 and m0
+//                 formed from the modulation and the timestep embedding
+//   time_embed    the time MLP and projection on one timestep, sinusoid included
+//
+// bf16_linear on contiguous rows of whole 128-byte stages runs on the GEMM of
+// fp8.hip, and large bf16-weight heads on the LDS-staged kernel below.  The other
+// MFMA kernels here read their operands straight from global memory (L2), without
+// LDS staging, for odd layouts, few rows or fp32 weights: one wave's 32-row operand
+// slice is re-read by at most two waves of its workgroup.  Lanes 0-31 of an MFMA
+// operand hold rows 0-31 of k-slice [k0, k0+8), lanes 32-63 the same rows at
+// [k0+8, k0+16): a k index is paired the same way in A and W, so the sum over k is
+// the GEMM's.
 #include "common.h"
 
 namespace srdit {

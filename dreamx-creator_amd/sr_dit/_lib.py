@@ -292,8 +292,9 @@ def fp8_linear(x, w, w_scale, bias, rowwise):
     N = w.shape[0]
     if w.dtype != torch.float8_e4m3fn or w.dim() != 2 or w.shape[1] != K or not w.is_contiguous():
         raise ValueError(f"fp8_linear: w must be a contiguous float8_e4m3fn [N, {K}] tensor")
-    if w_scale.dtype != torch.float32 or not w_scale.is_contiguous():
-        raise ValueError("fp8_linear: w_scale must be contiguous float32")
+    if w_scale.dtype != torch.float32:
+        raise ValueError("fp8_linear: w_scale must be float32")
+    w_scale = w_scale.contiguous()
     if bias is not None and (bias.dtype != torch.bfloat16 or bias.numel() != N
                              or not bias.is_contiguous()):
         raise ValueError(f"fp8_linear: bias must be {N} contiguous bf16 values")
@@ -608,7 +609,7 @@ def head_linear_fits(rows, w, mod, e):
     return (w.dtype == torch.bfloat16 and K % 64 == 0 and K <= 4096
             and (N <= 64 or rows * -(-N // 192) >= 2560)
             and mod.dtype in _DENSE_W_CODES and mod.numel() == 2 * K and mod.is_contiguous()
-            and e.dtype == torch.float32 and e.numel() == K and e.is_contiguous())
+            and e.dtype == torch.float32 and tuple(e.shape) == (1, K) and e.is_contiguous())
 
 
 def head_linear(a, mod, e, w, bias, out):
@@ -654,7 +655,7 @@ def gemv_f32(x, w, bias, out):
 def time_embed_fits(t, lins):
     """Whether ``time_embed`` takes this timestep and these three Linears (the time
     MLP's two and the projection)."""
-    if t.dtype != torch.float32 or t.numel() != 1 or not t.is_cuda:
+    if t.dtype != torch.float32 or tuple(t.shape) != (1,) or not t.is_cuda:
         return False
     dt, dim = lins[0].weight.dtype, lins[0].out_features
     if dt not in _DENSE_W_CODES or lins[0].in_features % 8 or lins[0].in_features > 2048 \
